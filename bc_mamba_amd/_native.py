@@ -114,6 +114,9 @@ SIGNATURES = {
     "bcm_restore_proj_bwd_workspace_bytes": (c_i64, [c_i64, c_i64, c_i64, c_i64]),
     "bcm_restore_proj_bwd": (c_i32, [c_p, c_p, c_i64, c_p, c_i64, c_p, c_i64, c_i64, c_i64, c_p, c_i64, c_p, c_p,
                                      c_p, c_i64, c_p]),
+    "bcm_gemm_f32_workspace_bytes": (c_i64, [c_i64, c_i64, c_i64]),
+    "bcm_gemm_f32": (c_i32, [c_p, c_i32, c_i64, c_p, c_i32, c_i64, c_p, c_i64, c_i64, c_i64, c_p, c_i64, c_p, c_i64,
+                             c_p]),
 }
 
 RESTORE_BWD_NOALLOC_MAX_TILES = 699040  # BCM_RESTORE_BWD_NOALLOC_MAX_TILES of the header

@@ -268,7 +268,7 @@ class _IndexedRestoreProjFn(torch.autograd.Function):
             return restore_dense_cuda_nodecay.restore_proj_fwd_indexed(y_flat, event_index, n_ch, dim, seqlen,
                                                                         weight, bias)
         z = restore_dense_cuda_nodecay.restore_fwd_indexed(y_flat, event_index, n_ch, dim, seqlen)
-        return F.linear(z, weight, bias)
+        return projections.mm(z.view(-1, dim), weight.t(), bias).view(z.size(0), seqlen, weight.size(0))
 
     @staticmethod
     def backward(ctx, dout):

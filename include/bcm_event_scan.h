@@ -536,6 +536,23 @@ int bcm_restore_proj_bwd(const float* dout, const float* y, int64_t n_events,
                          float* dweight, void* workspace, int64_t workspace_bytes,
                          bcm_stream_t stream);
 
+/* ---- (4) fp32 products of the token projections ------------------------- */
+/* C[m][n] = sum over k of A(m, k) B(n, k) + bias[n], fp32 in and out: the
+ * products of in_proj, out_proj and prob_head (e_model.py:419-506) and of
+ * their gradients, at fp32 accuracy on the fp16 matrix cores (each value
+ * split into two scaled fp16 values, fp32 sums; infinities and NaN as in a
+ * plain fp32 product). A(m, k) is a[m * lda + k] when a_k_contiguous, else
+ * a[k * lda + m]; B alike over n; (a_k_contiguous, b_k_contiguous) = (0, 1)
+ * has no form. bias may be NULL. Each operand's span, padded by 32 rows, and
+ * C's stay below 2 GiB. A workspace of bcm_gemm_f32_workspace_bytes lets few
+ * and long sums (a weight gradient) be split over the chip, partials summed
+ * in a fixed order; without it (or with a bias) they are not split. */
+int64_t bcm_gemm_f32_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int bcm_gemm_f32(const float* a, int a_k_contiguous, int64_t lda, const float* b,
+                 int b_k_contiguous, int64_t ldb, const float* bias, int64_t M,
+                 int64_t N, int64_t K, float* c, int64_t ldc, void* workspace,
+                 int64_t workspace_bytes, bcm_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -185,3 +185,26 @@ def test_split_k_projections_match_torch():
     (wi2 @ h2.t()).backward(g)
     assert torch.allclose(wi.grad, wi2.grad, rtol=1e-4, atol=1e-4 * wi2.grad.abs().max().item())
     assert torch.allclose(h.grad, h2.grad, rtol=1e-5, atol=1e-5)
+
+
+def test_projection_kernel_rule_and_argument_checks():
+    """bcm_gemm_f32 refuses what it has no form for before any launch; CPU
+    tensors stay with torch."""
+    from bc_mamba_amd import _native as nat
+    from bc_mamba_amd import projections as pj
+    a, b = torch.randn(5, 7), torch.randn(7, 3)
+    assert pj._kernel_form(a, b) is None and torch.equal(pj.mm(a, b), a @ b)
+    lib = nat.lib()
+    ok = [16, 1, 7, 16, 0, 3, None, 5, 3, 7, 16, 3, None, 0, None]
+
+    def rc(**kw):
+        return lib.bcm_gemm_f32(*[kw.get(f"p{i}", v) for i, v in enumerate(ok)])
+
+    assert rc(p9=0) == 1 and "invalid sizes" in lib.bcm_last_error().decode()
+    assert rc(p0=None) == 1 and "null pointer" in lib.bcm_last_error().decode()
+    assert rc(p2=6) == 1 and "leading dimension" in lib.bcm_last_error().decode()
+    assert rc(p1=0, p4=1, p5=7) == 1 and "no form" in lib.bcm_last_error().decode()
+    assert rc(p2=2 ** 28) == 1 and "too large" in lib.bcm_last_error().decode()
+    assert rc(p7=0) == 0
+    assert lib.bcm_gemm_f32_workspace_bytes(0, 4, 4) == 0
+    assert lib.bcm_gemm_f32_workspace_bytes(51200, 512, 256) == 0  # enough tiles: not split
