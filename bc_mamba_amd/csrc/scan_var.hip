@@ -11,22 +11,28 @@
 // :1087-1112 (constant B / C sums), selective_scan.cpp:1085-1090 (dB / dC
 // mirror the B / C layout).
 //
-// MI355X design: one workgroup per model channel d (its waves take the
-// channels b·dim + d, so dA, ddt, dD and the constant-B/C sums reduce in LDS
-// in a fixed order: no atomics, deterministic). A channel runs in passes of
-// 128 events: 16 lanes (one DPP row) × 8 consecutive events per lane. Per
+// MI355X design: one workgroup per model channel d (its channels are b·dim + d,
+// so dA, ddt, dD and the constant-B/C sums reduce in LDS in a fixed order: no
+// atomics, deterministic). A channel runs in passes of 128 events: 16 lanes
+// (one DPP row) × 8 consecutive events per lane, four channels a wave. Per
 // pass and state a lane folds its 8 items, the row combines the folds with
 // the DPP scan of scan_group.hpp, and a second register pass produces the
 // states; (decay product, h) and the backward's a·dh carry to the next pass
-// through LDS. B and C are read per (state, event) straight from global
-// memory: 8 consecutive events per lane, 512 contiguous bytes per row. The
-// backward reads the forward states from a workspace [dstate, E] that a
-// forward pass over the same inputs writes first, so it needs no chunk
-// re-seeding. These modes are not used by the BC_mamba block; the kernels
-// aim at correctness at memory speed, not at the depthwise path's VALU tuning.
+// through LDS. The backward reads the forward states from a workspace
+// [dstate, E] that a forward pass over the same inputs writes first.
+//
+// A channel is a chain of passes × states, and each link waits on its B and C
+// from memory. Two things shorten it: the waves a workgroup has to spare (8,
+// less one per four channels) take a share of the states each, their sums
+// over the states meeting in LDS once a pass, and every link's operands are
+// sent for one link ahead, as 16-byte loads. 153 000 events of 768 channels,
+// dstate 16, fp32 with z: forward 94 -> 37 us, backward 159 -> 80 us
+// (16 forward waves of 2 states each: 44; without the events one pass ahead: 42
+// and 90).
 #include "bcm_common.hpp"
 #include "scan_group.hpp"
 
+#include <algorithm>
 #include <climits>
 
 namespace bcm {
@@ -35,74 +41,143 @@ namespace {
 constexpr int kVG = 16;              // lanes per channel group
 constexpr int kVR = 8;               // consecutive events per lane
 constexpr int kVPass = kVG * kVR;    // events per pass
-constexpr int kVThreads = 256;       // 4 waves, 16 channel groups
+constexpr int kVWaves = 8;           // most waves of a workgroup
+constexpr int kVThreads = kVWaves * kWave;
 constexpr int kXChunk = 2048;        // events per saved-state chunk (selective_scan.cpp:795)
 constexpr float kLog2eV = 1.4426950408889634f;
 static_assert(kXChunk % kVPass == 0, "passes must tile the saved-state chunks");
 
-struct VarLds {
-  int N, nslots;
-  bool bwd;
-  int64_t bytes() const {
-    return 4ll * (4ll * N + (int64_t)nslots * (bwd ? (N + 3 * N + 3) : 2 * N));
+// Shape of a workgroup: nq waves side by side over the channels (four each),
+// ns waves behind one another over the states (wave w: channels w % nq,
+// states w / nq, w / nq + ns, ...).
+struct VarShape {
+  int nq, ns;
+  int waves() const { return nq * ns; }
+  int slots() const { return nq * (kWave / kVG); }
+  // floats of LDS: A log2e, A, constant B, constant C; per slot the carries
+  // and (backward) the gradient accumulators; two stages of the waves'
+  // partial sums over their states
+  int64_t bytes(int N, bool bwd) const {
+    const int64_t part = ns > 1 ? 2ll * waves() * kWave * kVR * (bwd ? 2 : 1) : 0;
+    return 4ll * (4ll * N + (int64_t)slots() * (bwd ? N + 3 * N + 3 : 2 * N) + part);
   }
 };
 
-// Element offsets of one operand for the 8 items of a lane in a pass:
-// off(s, r) = base[r] + s * sstride, valid when ok[r].
-struct BcOperand {
+// One operand's values for the 8 items of a lane, for one state: element
+// base + s * sstride + r. vec: the whole group of 8 lies in the operand's
+// memory (16-byte loads; the values of items past the channel's end are
+// not used); otherwise item by item.
+struct VarOperand {
   const float* p;
-  int64_t base[kVR];
-  int64_t sstride;
-  bool ok[kVR];
+  int64_t base;
+  bool vec, on;
+
+  // per_event: one value per event; otherwise the operand has no such values
+  __device__ __forceinline__ void at(const float* ptr, bool per_event, const bcm_scan_bc& bc, bool tiled, int64_t e_first,
+                                     int pos, int n, int64_t tile0, int N, int64_t E) {
+    p = ptr;
+    on = per_event && pos < n;
+    if (!per_event) return;
+    if (!tiled) {
+      base = e_first;
+      vec = __all(!on || e_first + kVR <= E);
+    } else {
+      const int T = bc.tile_chunk_size;
+      const int64_t tile = tile0 + pos / T;
+      base = tile * N * (int64_t)T + pos % T;
+      vec = __all(!on || (T % kVR == 0 && tile >= 0 && tile < bc.n_tiles));
+    }
+  }
+  // where vec is false: the offset of item r, or -1
+  static __device__ __forceinline__ int64_t item(int r, const bcm_scan_bc& bc, bool tiled, int64_t e_first, int pos, int n,
+                                                 int64_t tile0, int N) {
+    pos = opaque(pos);  // worked out where it is used: offsets of 8 items for each operand would not fit the registers
+    if (pos + r >= n) return -1;
+    if (!tiled) return opaque(e_first) + r;
+    const int T = bc.tile_chunk_size;
+    const int64_t t = tile0 + (pos + r) / T;
+    return t >= 0 && t < bc.n_tiles ? t * N * (int64_t)T + (pos + r) % T : -1;
+  }
+  template <typename F> __device__ __forceinline__ void load(float (&v)[kVR], int64_t so, F&& it) const {
+#pragma unroll
+    for (int r = 0; r < kVR; ++r) v[r] = 0.0f;
+    if (vec) {
+      if (on) __builtin_memcpy(v, p + so + base, sizeof(v));
+    } else {
+#pragma unroll
+      for (int r = 0; r < kVR; ++r) {
+        const int64_t o = on ? it(r) : -1;
+        if (o >= 0) v[r] = p[so + o];
+      }
+    }
+  }
+  template <typename F> __device__ __forceinline__ void store(const float (&v)[kVR], int64_t so, int items, F&& it) const {
+    float* q = const_cast<float*>(p) + so;
+    if (vec && items >= kVR) {
+      __builtin_memcpy(q + base, v, sizeof(v));
+    } else {
+#pragma unroll
+      for (int r = 0; r < kVR; ++r) {
+        const int64_t o = r < items ? it(r) : -1;
+        if (o >= 0) q[o] = v[r];
+      }
+    }
+  }
 };
 
-__device__ __forceinline__ void bc_offsets(BcOperand& o, const float* ptr, bool per_event, bool tiled,
-                                           int64_t row_stride, int64_t e_first, int pos_first, int n,
-                                           int64_t tile0, int T, int N, int64_t n_tiles) {
-  o.p = ptr;
-  o.sstride = tiled ? T : row_stride;
+// The raw values of a lane's 8 events of one pass from one stream (on: the
+// lane has events; vec: 16-byte loads, all 8 lie in the stream; items past the
+// channel's end are not used).
+template <typename T> struct VarEvents {
+  T v[kVR];
+  __device__ __forceinline__ void load(const T* p, int64_t e, bool on, bool vec, int64_t E) {
+    if (vec) {
+      if (on) __builtin_memcpy(v, p + e, sizeof(v));
+    } else {
 #pragma unroll
-  for (int r = 0; r < kVR; ++r) {
-    const int pos = pos_first + r;
-    bool ok = per_event && pos < n;
-    int64_t base = e_first + r;
-    if (tiled) {
-      const int64_t tile = tile0 + pos / T;
-      ok = ok && tile >= 0 && tile < n_tiles;
-      base = (tile * N) * (int64_t)T + pos % T;
+      for (int r = 0; r < kVR; ++r) v[r] = p[max((int64_t)0, min(e + r, E - 1))];
     }
-    o.ok[r] = ok;
-    o.base[r] = ok ? base : 0;
   }
-}
+};
 
-__device__ __forceinline__ float bc_load(const BcOperand& o, int r, int s) {
-  return o.ok[r] ? o.p[o.base[r] + (int64_t)s * o.sstride] : 0.0f;
+// Most passes of the workgroup's channels (their waves keep step at the
+// partial sums).
+__device__ __forceinline__ int var_passes(int np, int ns, int* s_np) {
+  const int npw = wave_max_dpp(np);
+  if (ns == 1) return npw;
+  __syncthreads();
+  if (threadIdx.x == 0) *s_np = 0;
+  __syncthreads();
+  if (lane_id() == 0) atomicMax(s_np, npw);
+  __syncthreads();
+  return *s_np;
 }
 
 }  // namespace
 
 template <typename T, bool HAS_Z, bool VB, bool VC>
-__global__ __launch_bounds__(kVThreads) void k_scan_var_fwd(const bcm_scan_args a, const bcm_scan_bc bc,
+__global__ __launch_bounds__(kVThreads) void k_scan_var_fwd(const bcm_scan_args a, const bcm_scan_bc bc, int nq, int ns,
                                                             float* __restrict__ hws) {
   using Ops = Grp<kVG>;
   const int N = a.dstate;
   const int d = blockIdx.x;
-  const int nw = blockDim.x / kWave;
   const int wave = threadIdx.x / kWave, lane = lane_id();
   const int grp = lane / kVG, j = lane % kVG;
-  const int nslots = nw * (kWave / kVG);
-  const int slot = wave * (kWave / kVG) + grp;
+  const int wq = wave % nq, ws = wave / nq;
+  const int nslots = nq * (kWave / kVG);
+  const int slot = wq * (kWave / kVG) + grp;
+  const int nthr = nq * ns * kWave;
   const bool tiled = bc.layout == BCM_BC_TILED;
 
   extern __shared__ float smem[];
+  __shared__ int s_np;
   float* sAl = smem;
   float* sB = sAl + N;  // constant B / C column of d
   float* sC = sB + N;
-  float* carry = sC + 2 * N + slot * 2 * N;  // [P(N), h(N)] at the end of the previous pass
+  float* carry = sC + 2 * N + slot * 2 * N;   // [P(N), h(N)] at the end of the previous pass
+  float* part = sC + 2 * N + nslots * 2 * N;  // [2][waves][8][64] partial y
 
-  for (int s = threadIdx.x; s < N; s += blockDim.x) {
+  for (int s = threadIdx.x; s < N; s += nthr) {
     sAl[s] = a.A[(int64_t)d * N + s] * kLog2eV;
     sB[s] = VB ? 0.0f : bc.B[(int64_t)s * bc.b_row_stride + d];
     sC[s] = VC ? 0.0f : bc.C[(int64_t)s * bc.c_row_stride + d];
@@ -127,42 +202,73 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_fwd(const bcm_scan_args 
     // events stay inside [0, E) whatever cu_seqlens holds
     const int n = (act && e0 >= 0) ? (int)max((int64_t)0, min((int64_t)a.cu_seqlens[ch + 1], E) - e0) : 0;
     const int np = (n + kVPass - 1) / kVPass;
-    const int npw = wave_max_dpp(np);
+    const int npw = var_passes(np, ns, &s_np);
     const int64_t tile0 = (tiled && act) ? (int64_t)bc.tile_offsets[ch] : 0;
+    VarOperand ob, oc;
+    float bn[kVR], cn[kVR];  // the next link's B and C
+    int ppos = 0;      // the lane's first event of the pass that is fetched for
+    auto operands = [&](int p) {
+      ppos = p * kVPass + j * kVR;
+      ob.at(bc.B, VB, bc, tiled, (int64_t)e0 + ppos, ppos, n, tile0, N, E);
+      oc.at(bc.C, VC, bc, tiled, (int64_t)e0 + ppos, ppos, n, tile0, N, E);
+    };
+    auto item = [&](int r) { return VarOperand::item(r, bc, tiled, (int64_t)e0 + ppos, ppos, n, tile0, N); };
+    auto fetch = [&](int s) {
+      if (VB) ob.load(bn, s * (tiled ? (int64_t)bc.tile_chunk_size : bc.b_row_stride), item);
+      if (VC) oc.load(cn, s * (tiled ? (int64_t)bc.tile_chunk_size : bc.c_row_stride), item);
+    };
+    // the next pass's u, k and z, on their way like the operands
+    VarEvents<T> un, zn;
+    VarEvents<int32_t> kn;
+    auto events = [&](int p) {
+      const int64_t e = (int64_t)e0 + p * kVPass + j * kVR;
+      const bool on = p * kVPass + j * kVR < n, vec = __all(!on || e + kVR <= E);
+      un.load(u, e, on, vec, E);
+      kn.load(a.k, e, on, vec, E);
+      if (HAS_Z && out) zn.load(z, e, on, vec, E);
+    };
+    operands(0);
+    if (npw > 0) {
+      events(0);
+      if (ws < N) fetch(ws);
+    }
     for (int p = 0; p < npw; ++p) {
       const int pos0 = p * kVPass + j * kVR;
-      float uu[kVR], dl[kVR], dlu[kVR], y[kVR];
-      bool valid[kVR];
+      const int64_t eb = (int64_t)e0 + pos0;
+      const int items = max(0, min(kVR, n - pos0));
+      float dl[kVR], dlu[kVR], y[kVR], zv[kVR];
 #pragma unroll
       for (int r = 0; r < kVR; ++r) {
-        valid[r] = pos0 + r < n;
-        const int64_t e = (int64_t)e0 + pos0 + r;
-        uu[r] = valid[r] ? to_f(u[e]) : 0.0f;
-        const int kk = valid[r] ? a.k[e] : 1;
-        dl[r] = valid[r] ? fmaf(dti, (float)(kk - 1), dta) : 0.0f;
-        dlu[r] = dl[r] * uu[r];
-        y[r] = Dv * uu[r];
+        const float uu = r < items ? to_f(un.v[r]) : 0.0f;
+        dl[r] = r < items ? fmaf(dti, (float)(kn.v[r] - 1), dta) : 0.0f;
+        dlu[r] = dl[r] * uu;
+        y[r] = ws == 0 ? Dv * uu : 0.0f;
+        if (HAS_Z) zv[r] = r < items ? to_f(zn.v[r]) : 0.0f;
       }
-      BcOperand ob, oc;
-      bc_offsets(ob, bc.B, VB, tiled, bc.b_row_stride, (int64_t)e0 + pos0, pos0, n, tile0, bc.tile_chunk_size, N,
-                 bc.n_tiles);
-      bc_offsets(oc, bc.C, VC, tiled, bc.c_row_stride, (int64_t)e0 + pos0, pos0, n, tile0, bc.tile_chunk_size, N,
-                 bc.n_tiles);
+      if (p + 1 < npw) events(p + 1);
       // the pass that holds the last event of a saved-state chunk (or of the channel)
       const int pass_end = min(n, (p + 1) * kVPass);
       const bool save_x = a.x && p < np && (pass_end % kXChunk == 0 || pass_end == n);
       const int xc = (pass_end - 1) / kXChunk;
 #pragma unroll 1
-      for (int s = 0; s < N; ++s) {
+      for (int s = ws; s < N; s += ns) {
         const float Al = sAl[s];
         float av[kVR], xv[kVR], cv[kVR];
+#pragma unroll
+        for (int r = 0; r < kVR; ++r) {
+          xv[r] = r < items ? (VB ? bn[r] : sB[s]) * dlu[r] : 0.0f;
+          cv[r] = VC ? cn[r] : sC[s];
+        }
+        if (s + ns < N) {  // the next link: the wave's next state, or its first one of the next pass
+          fetch(s + ns);
+        } else if (p + 1 < npw) {
+          operands(p + 1);
+          fetch(ws);
+        }
         float P = 1.0f, H = 0.0f;
 #pragma unroll
         for (int r = 0; r < kVR; ++r) {
-          av[r] = valid[r] ? decay(dl[r] * Al) : 1.0f;
-          const float bv = VB ? bc_load(ob, r, s) : sB[s];
-          xv[r] = valid[r] ? bv * dlu[r] : 0.0f;
-          cv[r] = VC ? bc_load(oc, r, s) : sC[s];
+          av[r] = r < items ? decay(dl[r] * Al) : 1.0f;
           H = fmaf(av[r], H, xv[r]);
           P *= av[r];
         }
@@ -171,11 +277,22 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_fwd(const bcm_scan_args 
         const float P0 = p > 0 ? carry[s] : 1.0f;
         const float hend = fmaf(P, h0, H);
         float h = Ops::prev(hend, h0);
+        float hv[kVR];
 #pragma unroll
         for (int r = 0; r < kVR; ++r) {
           h = fmaf(av[r], h, xv[r]);
-          y[r] = fmaf(cv[r], h, y[r]);
-          if (hws && valid[r]) hws[(int64_t)s * E + e0 + pos0 + r] = h;
+          y[r] = r < items ? fmaf(cv[r], h, y[r]) : 0.0f;
+          hv[r] = h;
+        }
+        if (hws) {
+          float* q = hws + (int64_t)s * E + eb;
+          if (items == kVR) {
+            __builtin_memcpy(q, hv, sizeof(hv));
+          } else {
+#pragma unroll
+            for (int r = 0; r < kVR; ++r)
+              if (r < items) q[r] = hv[r];
+          }
         }
         if (j == kVG - 1 && p < np) {
           carry[s] = P0 * P;
@@ -188,20 +305,32 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_fwd(const bcm_scan_args 
         }
       }
       if (out) {
+        int r0 = 0, nr = kVR;
+        if (ns > 1) {  // the waves' sums over their states: each wave adds up kVR / ns of the lane's items
+          float* pp = part + (p & 1) * nq * ns * kWave * kVR;
+#pragma unroll
+          for (int r = 0; r < kVR; ++r) pp[(wave * kVR + r) * kWave + lane] = y[r];
+          __syncthreads();
+          nr = kVR / ns;
+          r0 = ws * nr;
+#pragma unroll
+          for (int r = 0; r < kVR; ++r) {
+            if (r < r0 || r >= r0 + nr) continue;
+            float v = 0.0f;
+            for (int q = 0; q < ns; ++q) v += pp[((q * nq + wq) * kVR + r) * kWave + lane];
+            y[r] = v;
+          }
+        }
 #pragma unroll
         for (int r = 0; r < kVR; ++r) {
-          if (!valid[r]) continue;
-          const int64_t e = (int64_t)e0 + pos0 + r;
-          out[e] = from_f<T>(y[r]);
-          if (HAS_Z) {
-            const float zv = to_f(z[e]);
-            out_z[e] = from_f<T>(y[r] * (zv / (1.0f + __expf(-zv))));
-          }
+          if (r >= items || r < r0 || r >= r0 + nr) continue;
+          out[eb + r] = from_f<T>(y[r]);
+          if (HAS_Z) out_z[eb + r] = from_f<T>(y[r] * (zv[r] / (1.0f + __expf(-zv[r]))));
         }
       }
     }
     // saved-state chunks past the channel's end keep the reference's zero state
-    if (act && a.x) {
+    if (act && a.x && ws == 0) {
       const int have = (n + kXChunk - 1) / kXChunk;
       for (int c = have; c < nck; ++c)
         for (int s = j; s < 2 * N; s += kVG) a.x[(ch * nck + c) * 2 * N + s] = 0.0f;
@@ -210,20 +339,22 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_fwd(const bcm_scan_args 
 }
 
 template <typename T, bool HAS_Z, bool VB, bool VC>
-__global__ __launch_bounds__(kVThreads) void k_scan_var_bwd(const bcm_scan_args a, const bcm_scan_bc bc,
+__global__ __launch_bounds__(kVThreads) void k_scan_var_bwd(const bcm_scan_args a, const bcm_scan_bc bc, int nq, int ns,
                                                             const float* __restrict__ hws) {
   using Ops = Grp<kVG>;
   const int N = a.dstate;
   const int d = blockIdx.x;
-  const int nw = blockDim.x / kWave;
   const int wave = threadIdx.x / kWave, lane = lane_id();
   const int grp = lane / kVG, j = lane % kVG;
-  const int nslots = nw * (kWave / kVG);
-  const int slot = wave * (kWave / kVG) + grp;
+  const int wq = wave % nq, ws = wave / nq;
+  const int nslots = nq * (kWave / kVG);
+  const int slot = wq * (kWave / kVG) + grp;
+  const int nthr = nq * ns * kWave;
   const bool tiled = bc.layout == BCM_BC_TILED;
   const int NA = 3 * N + 3;  // per slot: dA, constant dB, constant dC, ddt_idle, ddt_active, dD
 
   extern __shared__ float smem[];
+  __shared__ int s_np;
   float* sAl = smem;
   float* sA = sAl + N;
   float* sB = sA + N;
@@ -231,15 +362,16 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_bwd(const bcm_scan_args 
   float* cdh = sC + N + slot * N;                       // a·dh of the first event of the later pass
   float* sacc = sC + N + nslots * N;                    // [nslots][NA]
   float* cacc = sacc + slot * NA;
+  float* part = sacc + nslots * NA;                     // [2][waves][16][64] partial du, dΔ
 
-  for (int s = threadIdx.x; s < N; s += blockDim.x) {
+  for (int s = threadIdx.x; s < N; s += nthr) {
     const float Av = a.A[(int64_t)d * N + s];
     sA[s] = Av;
     sAl[s] = Av * kLog2eV;
     sB[s] = VB ? 0.0f : bc.B[(int64_t)s * bc.b_row_stride + d];
     sC[s] = VC ? 0.0f : bc.C[(int64_t)s * bc.c_row_stride + d];
   }
-  for (int i = threadIdx.x; i < nslots * NA; i += blockDim.x) sacc[i] = 0.0f;
+  for (int i = threadIdx.x; i < nslots * NA; i += nthr) sacc[i] = 0.0f;
   __syncthreads();
 
   const float dti = a.dt_idle[d], dta = a.dt_active[d];
@@ -253,6 +385,7 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_bwd(const bcm_scan_args 
   const T* __restrict__ osv = static_cast<const T*>(a.out_saved);
   T* __restrict__ du_out = static_cast<T*>(a.du);
   T* __restrict__ dz_out = static_cast<T*>(a.dz);
+  const int nr = kVR / ns, r0 = ws * nr;  // the items of a lane whose sums over the states this wave completes
 
   for (int b0 = 0; b0 < n_per_d; b0 += nslots) {
     const int b = b0 + slot;
@@ -262,54 +395,93 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_bwd(const bcm_scan_args 
     // events stay inside [0, E) whatever cu_seqlens holds
     const int n = (act && e0 >= 0) ? (int)max((int64_t)0, min((int64_t)a.cu_seqlens[ch + 1], E) - e0) : 0;
     const int np = (n + kVPass - 1) / kVPass;
-    const int npw = wave_max_dpp(np);
+    const int npw = var_passes(np, ns, &s_np);
     const int64_t tile0 = (tiled && act) ? (int64_t)bc.tile_offsets[ch] : 0;
     float ddti_l = 0.0f, ddta_l = 0.0f, dD_l = 0.0f;
+    VarOperand ob, oc, oh;
+    float bn[kVR], cn[kVR], hn[kVR], hp0n;  // the next link's B, C and states
+    int ppos = 0;                            // the lane's first event of the pass that is fetched for
+    auto operands = [&](int p) {
+      ppos = p * kVPass + j * kVR;
+      ob.at(bc.B, VB, bc, tiled, (int64_t)e0 + ppos, ppos, n, tile0, N, E);
+      oc.at(bc.C, VC, bc, tiled, (int64_t)e0 + ppos, ppos, n, tile0, N, E);
+      oh.at(hws, true, bc, false, (int64_t)e0 + ppos, ppos, n, 0, N, E);
+    };
+    auto item = [&](int r) { return VarOperand::item(r, bc, tiled, (int64_t)e0 + ppos, ppos, n, tile0, N); };
+    auto fetch = [&](int s) {
+      if (VB) ob.load(bn, s * (tiled ? (int64_t)bc.tile_chunk_size : bc.b_row_stride), item);
+      if (VC) oc.load(cn, s * (tiled ? (int64_t)bc.tile_chunk_size : bc.c_row_stride), item);
+      oh.load(hn, s * E, [&](int r) { return VarOperand::item(r, bc, false, (int64_t)e0 + ppos, ppos, n, 0, N); });
+      // state before the lane's first item
+      hp0n = (oh.on && ppos > 0) ? hws[s * E + e0 + ppos - 1] : 0.0f;
+    };
+    VarEvents<T> un, gn;  // the next pass's u, k and dout
+    VarEvents<int32_t> kn;
+    auto events = [&](int p) {
+      const int64_t e = (int64_t)e0 + p * kVPass + j * kVR;
+      const bool on = p * kVPass + j * kVR < n, vec = __all(!on || e + kVR <= E);
+      un.load(u, e, on, vec, E);
+      kn.load(a.k, e, on, vec, E);
+      gn.load(dout, e, on, vec, E);
+    };
+    if (npw > 0) {
+      events(npw - 1);
+      operands(npw - 1);
+      if (ws < N) fetch(ws);
+    }
     for (int p = npw - 1; p >= 0; --p) {
       const int pos0 = p * kVPass + j * kVR;
       const int64_t eb = (int64_t)e0 + pos0;
+      const int items = max(0, min(kVR, n - pos0));
       float uu[kVR], dl[kVR], dlu[kVR], dov[kVR], du[kVR], ddl[kVR];
       int km1[kVR];
-      bool valid[kVR];
+      VarEvents<T> zz, oo;
+      if (HAS_Z) {
+        const bool on = items > 0, vec = __all(!on || eb + kVR <= E);
+        zz.load(z, eb, on, vec, E);
+        oo.load(osv, eb, on, vec, E);
+      }
 #pragma unroll
       for (int r = 0; r < kVR; ++r) {
-        valid[r] = pos0 + r < n;
-        const int64_t e = eb + r;
-        uu[r] = valid[r] ? to_f(u[e]) : 0.0f;
-        km1[r] = valid[r] ? a.k[e] - 1 : 0;
-        dl[r] = valid[r] ? fmaf(dti, (float)km1[r], dta) : 0.0f;
+        uu[r] = r < items ? to_f(un.v[r]) : 0.0f;
+        dov[r] = r < items ? to_f(gn.v[r]) : 0.0f;
+        km1[r] = r < items ? kn.v[r] - 1 : 0;
+        dl[r] = r < items ? fmaf(dti, (float)km1[r], dta) : 0.0f;
         dlu[r] = dl[r] * uu[r];
-        float g = valid[r] ? to_f(dout[e]) : 0.0f;
-        if (HAS_Z && valid[r]) {  // selective_scan_bwd_kernel.cuh:795-801
-          const float zv = to_f(z[e]), ov = to_f(osv[e]);
+        if (HAS_Z && r < items) {  // selective_scan_bwd_kernel.cuh:795-801
+          const float zv = to_f(zz.v[r]), ov = to_f(oo.v[r]);
           const float sg = 1.0f / (1.0f + __expf(-zv));
-          dz_out[e] = from_f<T>(g * ov * sg * (1.0f + zv * (1.0f - sg)));
-          g *= zv * sg;
+          if (ws == 0) dz_out[eb + r] = from_f<T>(dov[r] * ov * sg * (1.0f + zv * (1.0f - sg)));
+          dov[r] *= zv * sg;
         }
-        dov[r] = g;
-        du[r] = Dv * g;
+        du[r] = ws == 0 ? Dv * dov[r] : 0.0f;
         ddl[r] = 0.0f;
-        dD_l = fmaf(g, uu[r], dD_l);
+        if (ws == 0) dD_l = fmaf(dov[r], uu[r], dD_l);
       }
-      BcOperand ob, oc, odb, odc;
-      bc_offsets(ob, bc.B, VB, tiled, bc.b_row_stride, eb, pos0, n, tile0, bc.tile_chunk_size, N, bc.n_tiles);
-      bc_offsets(oc, bc.C, VC, tiled, bc.c_row_stride, eb, pos0, n, tile0, bc.tile_chunk_size, N, bc.n_tiles);
-      bc_offsets(odb, bc.dB, VB, tiled, bc.db_row_stride, eb, pos0, n, tile0, bc.tile_chunk_size, N, bc.n_tiles);
-      bc_offsets(odc, bc.dC, VC, tiled, bc.dc_row_stride, eb, pos0, n, tile0, bc.tile_chunk_size, N, bc.n_tiles);
+      if (p > 0) events(p - 1);
+      VarOperand odb, odc;
+      odb.at(bc.dB, VB, bc, tiled, eb, pos0, n, tile0, N, E);
+      odc.at(bc.dC, VC, bc, tiled, eb, pos0, n, tile0, N, E);
+      auto ditem = [&](int r) { return VarOperand::item(r, bc, tiled, eb, pos0, n, tile0, N); };
 #pragma unroll 1
-      for (int s = 0; s < N; ++s) {
+      for (int s = ws; s < N; s += ns) {
         const float Al = sAl[s], Av = sA[s];
-        const float* hs_ = hws + (int64_t)s * E;
         float av[kVR], bv[kVR], gv[kVR], hv[kVR];
+        const float hp0 = hp0n;
 #pragma unroll
         for (int r = 0; r < kVR; ++r) {
-          av[r] = valid[r] ? decay(dl[r] * Al) : 1.0f;
-          bv[r] = VB ? bc_load(ob, r, s) : sB[s];
-          const float cv = VC ? bc_load(oc, r, s) : sC[s];
-          gv[r] = valid[r] ? cv * dov[r] : 0.0f;
-          hv[r] = valid[r] ? hs_[eb + r] : 0.0f;
+          bv[r] = VB ? bn[r] : sB[s];
+          gv[r] = r < items ? (VC ? cn[r] : sC[s]) * dov[r] : 0.0f;
+          hv[r] = r < items ? hn[r] : 0.0f;
         }
-        const float hp0 = (valid[0] && pos0 > 0) ? hs_[eb - 1] : 0.0f;  // state before the lane's first item
+        if (s + ns < N) {  // the next link of the walk
+          fetch(s + ns);
+        } else if (p > 0) {
+          operands(p - 1);
+          fetch(ws);
+        }
+#pragma unroll
+        for (int r = 0; r < kVR; ++r) av[r] = r < items ? decay(dl[r] * Al) : 1.0f;
         // dh_i = C_i dout_i + a_{i+1} dh_{i+1}; the last lane of the group
         // takes the carry a·dh of the later pass (and a "next decay" of 1)
         const float anext = Ops::next(av[0], 1.0f);
@@ -324,29 +496,24 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_bwd(const bcm_scan_args 
         Ops::scan_down(Q, Ce);
         float dh = Ops::next(fmaf(Q, ec, Ce), ec);
         float dA_l = 0.0f, dBc_l = 0.0f, dCc_l = 0.0f;
+        float dbv[kVR], dcv[kVR];
 #pragma unroll
         for (int r = kVR - 1; r >= 0; --r) {
           const float al = r == kVR - 1 ? anext : av[r + 1];
           dh = fmaf(al, dh, gv[r]);
           const float hp = r > 0 ? hv[r - 1] : hp0;
-          const float t = valid[r] ? dh * av[r] * hp : 0.0f;
+          const float t = r < items ? dh * av[r] * hp : 0.0f;
           dA_l = fmaf(t, dl[r], dA_l);
-          const float dhb = valid[r] ? dh * bv[r] : 0.0f;
+          const float dhb = r < items ? dh * bv[r] : 0.0f;
           ddl[r] = fmaf(dhb, uu[r], fmaf(Av, t, ddl[r]));
           du[r] = fmaf(dhb, dl[r], du[r]);
-          const float dbv = valid[r] ? dh * dlu[r] : 0.0f;
-          const float dcv = dov[r] * hv[r];
-          if (VB) {
-            if (odb.ok[r]) const_cast<float*>(odb.p)[odb.base[r] + (int64_t)s * odb.sstride] = dbv;  // bc.dB
-          } else {
-            dBc_l += dbv;
-          }
-          if (VC) {
-            if (odc.ok[r]) const_cast<float*>(odc.p)[odc.base[r] + (int64_t)s * odc.sstride] = dcv;  // bc.dC
-          } else {
-            dCc_l += dcv;
-          }
+          dbv[r] = r < items ? dh * dlu[r] : 0.0f;
+          dcv[r] = dov[r] * hv[r];
+          dBc_l += dbv[r];
+          dCc_l += dcv[r];
         }
+        if (VB && odb.on) odb.store(dbv, s * (tiled ? (int64_t)bc.tile_chunk_size : bc.db_row_stride), items, ditem);
+        if (VC && odc.on) odc.store(dcv, s * (tiled ? (int64_t)bc.tile_chunk_size : bc.dc_row_stride), items, ditem);
         if (j == 0 && p < np) cdh[s] = av[0] * dh;  // dh of the pass's first event
         dA_l = Ops::sum(dA_l);
         if (!VB) dBc_l = Ops::sum(dBc_l);
@@ -357,9 +524,30 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_bwd(const bcm_scan_args 
           if (!VC) cacc[2 * N + s] += dCc_l;
         }
       }
+      if (ns > 1) {  // the waves' sums over their states
+        float* pp = part + (p & 1) * nq * ns * kWave * 2 * kVR;
+#pragma unroll
+        for (int r = 0; r < kVR; ++r) {
+          pp[(wave * 2 * kVR + r) * kWave + lane] = du[r];
+          pp[(wave * 2 * kVR + kVR + r) * kWave + lane] = ddl[r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kVR; ++r) {
+          if (r < r0 || r >= r0 + nr) continue;
+          float v = 0.0f, w = 0.0f;
+          for (int q = 0; q < ns; ++q) {
+            v += pp[((q * nq + wq) * 2 * kVR + r) * kWave + lane];
+            w += pp[((q * nq + wq) * 2 * kVR + kVR + r) * kWave + lane];
+          }
+          du[r] = v;
+          ddl[r] = w;
+        }
+      }
 #pragma unroll
       for (int r = 0; r < kVR; ++r) {
-        if (valid[r]) du_out[eb + r] = from_f<T>(du[r]);
+        if (r >= items || r < r0 || r >= r0 + nr) continue;
+        du_out[eb + r] = from_f<T>(du[r]);
         ddti_l = fmaf(ddl[r], (float)km1[r], ddti_l);
         ddta_l += ddl[r];
       }
@@ -367,14 +555,17 @@ __global__ __launch_bounds__(kVThreads) void k_scan_var_bwd(const bcm_scan_args 
     ddti_l = Ops::sum(ddti_l);
     ddta_l = Ops::sum(ddta_l);
     dD_l = Ops::sum(dD_l);
-    if (j == 0 && act) {
-      cacc[3 * N] += ddti_l;
-      cacc[3 * N + 1] += ddta_l;
-      cacc[3 * N + 2] += dD_l;
+    for (int q = 0; q < ns; ++q) {  // one wave of a slot after the other: a fixed order
+      if (ns > 1) __syncthreads();
+      if (q == ws && j == 0 && act) {
+        cacc[3 * N] += ddti_l;
+        cacc[3 * N + 1] += ddta_l;
+        cacc[3 * N + 2] += dD_l;
+      }
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < NA; i += blockDim.x) {
+  for (int i = threadIdx.x; i < NA; i += nthr) {
     float v = 0.0f;
     for (int q = 0; q < nslots; ++q) v += sacc[q * NA + i];  // fixed order: deterministic
     if (i < N) {
@@ -434,16 +625,29 @@ static int var_checks(const bcm_scan_args* ap, const bcm_scan_bc* bc, bool bwd, 
   return BCM_OK;
 }
 
+// Waves over the channels first, the rest over the states (a power of two of
+// them, at most one per state and item), as far as LDS allows.
+static VarShape var_shape(const bcm_scan_args& a, bool bwd) {
+  const int64_t per_d = (a.n_channels + a.dim - 1) / a.dim, quads = (per_d + 3) / 4;
+  VarShape v{(int)std::max<int64_t>(1, std::min<int64_t>(kVWaves, quads)), 1};
+  while (v.nq * v.ns * 2 <= kVWaves && v.ns * 2 <= kVR && v.ns * 2 <= a.dstate) v.ns *= 2;
+  const int64_t lds = max_lds_bytes() - 256;
+  while (v.bytes(a.dstate, bwd) > lds && v.ns > 1) v.ns /= 2;
+  while (v.bytes(a.dstate, bwd) > lds && v.nq > 1) --v.nq;
+  return v;
+}
+
 template <bool BWD, typename T, bool Z, bool VB, bool VC>
 static int var_launch(const bcm_scan_args& a, const bcm_scan_bc& bc, float* hws, hipStream_t s, const char* fn) {
-  const int nw = kVThreads / kWave;
-  const int64_t lds = VarLds{a.dstate, nw * (kWave / kVG), BWD}.bytes();
+  const VarShape v = var_shape(a, BWD);
+  const int64_t lds = v.bytes(a.dstate, BWD);
   if (lds > max_lds_bytes())
     return set_error(BCM_EINVAL, "%s: dstate %d needs %lld bytes of LDS", fn, a.dstate, (long long)lds);
+  const dim3 block((unsigned)(v.waves() * kWave));
   if (BWD)
-    hipLaunchKernelGGL((k_scan_var_bwd<T, Z, VB, VC>), dim3(a.dim), dim3(kVThreads), (size_t)lds, s, a, bc, hws);
+    hipLaunchKernelGGL((k_scan_var_bwd<T, Z, VB, VC>), dim3(a.dim), block, (size_t)lds, s, a, bc, v.nq, v.ns, hws);
   else
-    hipLaunchKernelGGL((k_scan_var_fwd<T, Z, VB, VC>), dim3(a.dim), dim3(kVThreads), (size_t)lds, s, a, bc, hws);
+    hipLaunchKernelGGL((k_scan_var_fwd<T, Z, VB, VC>), dim3(a.dim), block, (size_t)lds, s, a, bc, v.nq, v.ns, hws);
   return check_launch(fn);
 }
 
