@@ -11,16 +11,26 @@
 //   dx[b,d,t] = sum_k w[d,k] * g[b,d,t+(K-1)-k]   (terms past L vanish)
 //   dw[d,k]   = sum_{b,t} g[b,d,t] * x[b,d,t-(K-1)+k],  dbias[d] = sum_{b,t} g
 //
-// MI355X design: rows (b, d) of L steps are contiguous. Each thread takes 4
-// consecutive steps of one row, read and written as whole 16-byte (fp32) or
-// 8-byte (fp16/bf16) vectors when L is a multiple of 4, with the K-1 halo
-// steps from the neighbouring vectors (L1 hits), so a wave covers 256
-// contiguous steps. The backward recomputes g from x (no saved
-// pre-activation); workgroup (d, p) takes every P-th batch row of channel d
-// (P chosen to fill the chip), writes dx, and reduces its dw / dbias
-// partials in registers and LDS in a fixed order; a small kernel sums the P
-// partials in group order (deterministic, no atomics). HBM-bound: x and dout
-// read once, out / dx written once.
+// MI355X design: rows (b, d) of L steps are contiguous. A thread takes S
+// consecutive steps of one row (16 bytes in the forward, 8 steps in the
+// backward, where a third of the halo's g would be recomputed at 4), with the
+// halo steps from the neighbours' vectors (L1 hits). Rows start anywhere (L
+// odd): the vectors are wide loads at any element alignment, values beyond
+// the row's ends are masked, and only the tensor's own ends go element by
+// element. A row takes the next power of two of threads that covers it (a
+// longer row several workgroups), a workgroup as many rows as fit, so short
+// rows fill it. The backward recomputes g from x (no saved pre-activation);
+// workgroup (d, p) takes every P-th group of rows of channel d (P chosen to
+// fill the chip), writes dx, and reduces its dw / dbias partials in registers
+// and LDS in a fixed order; a small kernel sums the P partials in group
+// order (deterministic, no atomics). Bound by memory (x and dout read once, out
+// / dx written once) and, in 16 bits, as much by the VALU (exponentials,
+// reciprocals).
+// us before (elements one by one where L % 4, 4 steps a thread, a 64-bit
+// division and an IEEE reciprocal a step) and now, forward / backward:
+//   [16, 512, 1023] bf16  19.3 / 31.8 -> 13.4 / 23.3,  fp32  24.0 / 42.3 -> 13.4 / 23.4
+//   [16, 512, 1024] bf16  13.2 / 23.8 -> 12.5 / 21.0,  fp32  13.6 / 22.1 -> 13.4 / 23.4
+//   [64, 512, 64] bf16     4.8 / 23.7 ->  4.8 / 9.3
 #include "bcm_common.hpp"
 
 #include <algorithm>
@@ -29,96 +39,124 @@
 namespace bcm {
 
 constexpr int kConvMaxK = 8;
-constexpr int kConvSteps = 4;  // consecutive steps per thread
 constexpr int kConvMaxSplit = 64;  // batch groups of the backward
+constexpr int kConvS = 8;          // consecutive steps per thread in the backward (fewer recomputed halo steps)
+template <typename T> constexpr int kConvSF = 16 / (int)sizeof(T);  // in the forward: 16 bytes
 
-// x[t .. t+3] of a row as floats: one 16-byte (fp32) or 8-byte (fp16/bf16)
-// load when VEC (t a multiple of 4, rows aligned), zeros for t < 0 or t >= L
-// (whole vectors: L is a multiple of 4 then); else per element with bounds.
-template <typename T, bool VEC>
-__device__ __forceinline__ void load4(const T* __restrict__ r, int64_t t, int64_t L, float* v) {
-  if (VEC) {
-    if (t < 0 || t >= L) {
-      v[0] = v[1] = v[2] = v[3] = 0.0f;
-    } else if constexpr (sizeof(T) == 4) {
-      const float4 q = *reinterpret_cast<const float4*>(r + t);
-      v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
-    } else {
-      const uint2 q = *reinterpret_cast<const uint2*>(r + t);
-      const T* e = reinterpret_cast<const T*>(&q);
-      v[0] = to_f(e[0]); v[1] = to_f(e[1]); v[2] = to_f(e[2]); v[3] = to_f(e[3]);
-    }
-  } else {
+// N elements from p as floats: one vector load, any alignment.
+template <int N, typename T> __device__ __forceinline__ void conv_load(const T* p, float* v) {
+  T e[N];
+  __builtin_memcpy(e, p, sizeof(e));
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = (t + i >= 0 && t + i < L) ? to_f(r[t + i]) : 0.0f;
+  for (int i = 0; i < N; ++i) v[i] = to_f(e[i]);
+}
+// A thread's place in a row: the steps before and after its first step that
+// lie in the row, and in the tensor (vectors may read on into neighbouring
+// rows, the values are masked). Distances are cut at 2^20.
+struct ConvAt {
+  int before, after;    // in the row: t0, L - t0
+  int tbefore, tafter;  // in the tensor
+  __device__ __forceinline__ ConvAt(int64_t row0, int64_t t0, int64_t L, int64_t total) {
+    const int64_t cut = 1 << 20;
+    before = (int)min(t0, cut);
+    after = (int)min(L - t0, cut);
+    tbefore = (int)min(row0 + t0, cut);
+    tafter = (int)min(total - row0 - t0, cut);
+  }
+};
+// Steps t0 - PRE .. t0 + S + POST - 1 (p: step t0) as floats, zeros outside the row.
+template <int PRE, int S, int POST, typename T>
+__device__ __forceinline__ void conv_window(const T* p, const ConvAt& at, float* v) {
+  if (at.tbefore >= PRE && at.tafter >= S + POST) {
+#pragma unroll
+    for (int i = 0; i < PRE; i += 4) conv_load<4>(p - PRE + i, v + i);
+    conv_load<S>(p, v + PRE);
+#pragma unroll
+    for (int i = 0; i < POST; i += 4) conv_load<4>(p + S + i, v + PRE + S + i);
+  } else {  // at the tensor's ends
+#pragma unroll
+    for (int i = 0; i < PRE + S + POST; ++i) v[i] = to_f(p[max(-at.before, min(i - PRE, at.after - 1))]);
+  }
+  if (at.before < PRE || at.after < S + POST) {
+#pragma unroll
+    for (int i = 0; i < PRE + S + POST; ++i) v[i] = i - PRE >= -at.before && i - PRE < at.after ? v[i] : 0.0f;
   }
 }
-
-template <typename T, bool VEC>
-__device__ __forceinline__ void store4(T* __restrict__ r, int64_t t, int64_t L, const float* v) {
-  if (VEC) {
-    if constexpr (sizeof(T) == 4) {
-      *reinterpret_cast<float4*>(r + t) = make_float4(v[0], v[1], v[2], v[3]);
-    } else {
-      T e[4] = {from_f<T>(v[0]), from_f<T>(v[1]), from_f<T>(v[2]), from_f<T>(v[3])};
-      *reinterpret_cast<uint2*>(r + t) = *reinterpret_cast<const uint2*>(e);
-    }
+template <int N, typename T> __device__ __forceinline__ void conv_store(T* p, const ConvAt& at, const float* v) {
+  T e[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) e[i] = from_f<T>(v[i]);
+  if (at.after >= N) {
+    __builtin_memcpy(p, e, sizeof(e));
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (t + i < L) r[t + i] = from_f<T>(v[i]);
+    for (int i = 0; i < N; ++i)
+      if (i < at.after) p[i] = e[i];
   }
+}
+// 1 / (1 + e^-v): the reciprocal refined once (two fused steps), within one
+// unit in the last place of the division. An overflowed e^-v gives 0.
+__device__ __forceinline__ float conv_sigmoid(float v) {
+  const float q = fminf(1.0f + __expf(-v), 3.0e38f), r = __builtin_amdgcn_rcpf(q);
+  return fmaf(fmaf(-q, r, 1.0f), r, r);
+}
+template <typename T> __device__ __forceinline__ void store4(T* __restrict__ r, int64_t t, const float* v) {
+  T e[4] = {from_f<T>(v[0]), from_f<T>(v[1]), from_f<T>(v[2]), from_f<T>(v[3])};  // whole aligned vectors
+  if constexpr (sizeof(T) == 4) *reinterpret_cast<float4*>(r + t) = *reinterpret_cast<const float4*>(e);
+  else *reinterpret_cast<uint2*>(r + t) = *reinterpret_cast<const uint2*>(e);
 }
 
 // KM = 4: width exactly 4 (d_conv's default), straight-line code; KM = 8:
-// any width K <= 8 given at run time.
-template <typename T, bool SILU, bool VEC, int KM>
+// any width K <= 8 given at run time. lg: log2 of the threads of a row; nseg:
+// workgroups of a row (1 unless lg is 8).
+template <typename T, bool SILU, int KM>
 __global__ __launch_bounds__(256) void k_conv_fwd(const T* __restrict__ x, const float* __restrict__ w,
-                                                  const float* __restrict__ bias, T* __restrict__ out, int64_t rows,
-                                                  int D, int64_t L, int K_, int64_t chunks) {
+                                                  const float* __restrict__ bias, T* __restrict__ out, int B, int D,
+                                                  int64_t L, int K_, int lg, int nseg) {
   const int K = KM == 4 ? 4 : K_;
+  constexpr int S = kConvSF<T>;
   constexpr int PRE = (KM - 1 + 3) / 4 * 4;  // halo steps before t0, whole vectors
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= rows * chunks) return;
-  const int64_t row = gid / chunks;
-  const int64_t t0 = (gid - row * chunks) * kConvSteps;
-  const int d = (int)(row % D);
-  const T* xr = x + row * L;
+  const int seg = blockIdx.x % nseg, db = blockIdx.x / nseg;
+  const int d = db * (256 >> lg) + (threadIdx.x >> lg);
+  const int64_t t0 = ((int64_t)seg * 256 + (threadIdx.x & ((1 << lg) - 1))) * S;
+  if (d >= D || t0 >= L) return;
   float wk[KM];
 #pragma unroll
   for (int k = 0; k < KM; ++k) wk[k] = k < K ? w[(int64_t)d * K + k] : 0.0f;
   const float b0 = bias ? bias[d] : 0.0f;
-  // window x[t0-PRE .. t0+3] (xv[i] = x[t0-PRE+i])
-  float xv[PRE + 4];
+  for (int b = blockIdx.y; b < B; b += gridDim.y) {
+    const int64_t row0 = ((int64_t)b * D + d) * L;
+    const ConvAt at(row0, t0, L, (int64_t)B * D * L);
+    float xv[PRE + S];  // xv[i] = x[t0-PRE+i]
+    conv_window<PRE, S, 0>(x + row0 + t0, at, xv);
+    float o[S];
 #pragma unroll
-  for (int v = 0; v < PRE / 4 + 1; ++v) load4<T, VEC>(xr, t0 - PRE + 4 * v, L, xv + 4 * v);
-  float o[kConvSteps];
+    for (int s = 0; s < S; ++s) {
+      // step t0+s reads x[t0+s-(K-1)+k] = xv[PRE+s-(K-1)+k]
+      float pre = b0;
 #pragma unroll
-  for (int s = 0; s < kConvSteps; ++s) {
-    // step t0+s reads x[t0+s-(K-1)+k] = xv[PRE+s-(K-1)+k]
-    float pre = b0;
-#pragma unroll
-    for (int k = 0; k < KM; ++k)
-      if (k < K) pre = fmaf(wk[k], xv[PRE + s - (K - 1) + k], pre);
-    o[s] = SILU ? pre / (1.0f + __expf(-pre)) : pre;
+      for (int k = 0; k < KM; ++k)
+        if (k < K) pre = fmaf(wk[k], xv[PRE + s - (K - 1) + k], pre);
+      o[s] = SILU ? pre / (1.0f + __expf(-pre)) : pre;
+    }
+    conv_store<S>(out + row0 + t0, at, o);
   }
-  store4<T, VEC>(out + row * L, t0, L, o);
 }
 
-// Backward of a group of batch rows of channel d: workgroup (d, p) takes the
-// rows b = p, p + P, ... (P = gridDim.y); with P > 1 its dw / dbias partials
-// go to part[(p * D + d) * (K + 1) ...] for k_conv_bwd_reduce.
-template <typename T, bool SILU, bool VEC, int KM>
+// Backward of channel d's rows: a unit is one row's segment of 256 S steps
+// (nseg of them), or R = 256 >> lg whole rows side by side; workgroup (d, p)
+// takes the units p, p + P, ... (P = gridDim.y); with P > 1 its dw / dbias
+// partials go to part[(p * D + d) * (K + 1) ...] for k_conv_bwd_reduce.
+template <typename T, bool SILU, int KM>
 __global__ __launch_bounds__(256) void k_conv_bwd(const T* __restrict__ x, const float* __restrict__ w,
                                                   const float* __restrict__ bias, const T* __restrict__ dout,
                                                   T* __restrict__ dx, float* __restrict__ dw,
                                                   float* __restrict__ dbias, float* __restrict__ part, int B, int D,
-                                                  int64_t L, int K_) {
+                                                  int64_t L, int K_, int lg, int nseg, int64_t units) {
   const int K = KM == 4 ? 4 : K_;  // KM = 4: width exactly 4
-  constexpr int PRE = (KM - 1 + 3) / 4 * 4;       // halo steps before t0, whole vectors
-  constexpr int NG = kConvSteps + KM - 1;          // g at t0 .. t0+NG-1
-  constexpr int NGV = (NG + 3) / 4 * 4;            // ... in whole vectors
-  constexpr int NX = PRE + NGV;                    // x at t0-PRE .. t0+NGV-1
+  constexpr int S = kConvS;
+  constexpr int PRE = (KM - 1 + 3) / 4 * 4;  // halo steps before t0 and after t0 + S, whole vectors
+  constexpr int NG = S + KM - 1;             // g at t0 .. t0+NG-1
   __shared__ float s_red[kConvMaxK + 1][256 / kWave];
   const int d = blockIdx.x, p = blockIdx.y, P = gridDim.y;
   float wk[KM];
@@ -128,48 +166,45 @@ __global__ __launch_bounds__(256) void k_conv_bwd(const T* __restrict__ x, const
   float aw[kConvMaxK], ab = 0.0f;  // this thread's dw / dbias partials
 #pragma unroll
   for (int k = 0; k < kConvMaxK; ++k) aw[k] = 0.0f;
-  for (int b = p; b < B; b += P) {
-    const int64_t row = (int64_t)b * D + d;
-    const T* xr = x + row * L;
-    const T* gr = dout + row * L;
-    T* dxr = dx + row * L;
-    for (int64_t t0 = (int64_t)threadIdx.x * kConvSteps; t0 < L; t0 += (int64_t)blockDim.x * kConvSteps) {
-      float xv[NX], go[NGV];  // xv[i] = x[t0-PRE+i], go[i] = dout[t0+i]
+  for (int64_t u = p; u < units; u += P) {
+    const int64_t b = u / nseg * (256 >> lg) + (threadIdx.x >> lg);
+    const int64_t t0 = (u % nseg * 256 + (threadIdx.x & ((1 << lg) - 1))) * S;
+    if (b >= B || t0 >= L) continue;
+    const int64_t row0 = (b * D + d) * L;
+    const ConvAt at(row0, t0, L, (int64_t)B * D * L);
+    float xv[PRE + S + PRE], dv[S + PRE];  // xv[i] = x[t0-PRE+i], dv[i] = dout[t0+i]
+    conv_window<PRE, S, PRE>(x + row0 + t0, at, xv);
+    conv_window<0, S, PRE>(dout + row0 + t0, at, dv);
+    // g at steps t0+i (zero past L: dv is zero there)
+    float g[NG];
 #pragma unroll
-      for (int v = 0; v < NX / 4; ++v) load4<T, VEC>(xr, t0 - PRE + 4 * v, L, xv + 4 * v);
+    for (int i = 0; i < NG; ++i) {
+      float pre = b0;
 #pragma unroll
-      for (int v = 0; v < NGV / 4; ++v) load4<T, VEC>(gr, t0 + 4 * v, L, go + 4 * v);
-      // g at steps t0+i (zero past L: go is zero there)
-      float g[NG];
-#pragma unroll
-      for (int i = 0; i < NG; ++i) {
-        float pre = b0;
-#pragma unroll
-        for (int k = 0; k < KM; ++k)
-          if (k < K) pre = fmaf(wk[k], xv[PRE + i - (K - 1) + k], pre);
-        if (SILU) {
-          const float sg = 1.0f / (1.0f + __expf(-pre));
-          g[i] = go[i] * sg * fmaf(pre, 1.0f - sg, 1.0f);  // one rounding, in both conv backwards
-        } else {
-          g[i] = go[i];
-        }
+      for (int k = 0; k < KM; ++k)
+        if (k < K) pre = fmaf(wk[k], xv[PRE + i - (K - 1) + k], pre);
+      if (SILU) {
+        const float sg = conv_sigmoid(pre);
+        g[i] = dv[i] * sg * fmaf(pre, 1.0f - sg, 1.0f);  // one rounding, in both conv backwards
+      } else {
+        g[i] = dv[i];
       }
-      float o[kConvSteps];
-#pragma unroll
-      for (int s = 0; s < kConvSteps; ++s) {
-        float acc = 0.0f;
-#pragma unroll
-        for (int k = 0; k < KM; ++k)
-          if (k < K) acc = fmaf(wk[k], g[s + (K - 1) - k], acc);
-        o[s] = acc;
-        // dw[k] += g[t] x[t-(K-1)+k] over this thread's own steps (g is 0 past L)
-#pragma unroll
-        for (int k = 0; k < KM; ++k)
-          if (k < K) aw[k] = fmaf(g[s], xv[PRE + s - (K - 1) + k], aw[k]);
-        ab += g[s];
-      }
-      store4<T, VEC>(dxr, t0, L, o);
     }
+    float o[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      float acc = 0.0f;
+#pragma unroll
+      for (int k = 0; k < KM; ++k)
+        if (k < K) acc = fmaf(wk[k], g[s + (K - 1) - k], acc);
+      o[s] = acc;
+      // dw[k] += g[t] x[t-(K-1)+k] over this thread's own steps (g is 0 past L)
+#pragma unroll
+      for (int k = 0; k < KM; ++k)
+        if (k < K) aw[k] = fmaf(g[s], xv[PRE + s - (K - 1) + k], aw[k]);
+      ab += g[s];
+    }
+    conv_store<S>(dx + row0 + t0, at, o);
   }
   // fixed-order reduction: butterfly within each wave, then the waves in order
   const int wave = threadIdx.x / kWave, lane = lane_id();
@@ -316,7 +351,7 @@ __global__ __launch_bounds__(256) void k_conv_bwd_events(
           if (j < K) pre = fmaf(wk[j], xv[q][PRE + k - (K - 1) + j], pre);
         float gv = dv[q][k];
         if (SILU) {
-          const float sgm = 1.0f / (1.0f + __expf(-pre));
+          const float sgm = conv_sigmoid(pre);
           gv = dv[q][k] * sgm * fmaf(pre, 1.0f - sgm, 1.0f);  // as k_conv_bwd: one rounding
         }
         g[k] = ((nib[q] >> k) & 1u) ? gv : 0.0f;
@@ -348,7 +383,7 @@ __global__ __launch_bounds__(256) void k_conv_bwd_events(
             if (k < K) acc = fmaf(wk[k], gg[s + (K - 1) - k], acc);
           o[s] = acc;
         }
-        store4<T, true>(dr, t0, L, o);
+        store4(dr, t0, o);
       }
     }
     wave_sync();
@@ -388,10 +423,29 @@ __global__ __launch_bounds__(256) void k_conv_bwd_events_reduce(const float* __r
   else if (dbias) dbias[d] = v;
 }
 
-// Batch groups of the backward: enough workgroups to fill the chip.
-inline int conv_split(int64_t B, int64_t D) {
+// How rows are laid over workgroups: 2^lg threads a row (the next power of two
+// that covers it, at most 256), and nseg workgroups for a longer one.
+struct ConvShape {
+  int lg, R;
+  int64_t nseg;
+};
+static ConvShape conv_shape(int64_t L, int steps) {
+  const int64_t chunks = (L + steps - 1) / steps;
+  ConvShape c{0, 256, 1};
+  while (c.lg < 8 && (int64_t)(1 << c.lg) < chunks) ++c.lg;
+  c.R = 256 >> c.lg;
+  c.nseg = std::max<int64_t>(1, (chunks + 255) / 256);
+  return c;
+}
+static int64_t conv_units(int64_t B, int64_t L) {
+  const ConvShape c = conv_shape(L, kConvS);
+  return (B + c.R - 1) / c.R * c.nseg;
+}
+
+// Unit groups of the backward: enough workgroups to fill the chip.
+static int conv_split(int64_t B, int64_t D, int64_t L) {
   const int64_t want = (8 * (int64_t)device_cus() + D - 1) / D;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({B, want, (int64_t)kConvMaxSplit}));
+  return (int)std::max<int64_t>(1, std::min<int64_t>({conv_units(B, L), want, (int64_t)kConvMaxSplit}));
 }
 
 static int conv_checks(const char* fn, int dtype, int64_t B, int64_t D, int64_t L, int K) {
@@ -413,36 +467,30 @@ int bcm_causal_conv1d_fwd(const void* x, int dtype, const float* weight, const f
   if (rc) return rc;
   if (B == 0 || L == 0) return BCM_OK;
   if (!x || !weight || !out) return bcm::set_error(BCM_EINVAL, "%s: null pointer", fn);
-  const int64_t rows = B * D, chunks = (L + bcm::kConvSteps - 1) / bcm::kConvSteps;
-  const int64_t n = rows * chunks;
-  const dim3 grid((unsigned)((n + 255) / 256));
-  const bool vec = L % 4 == 0 && bcm::aligned16(x) && bcm::aligned16(out);
+  const bcm::ConvShape c = bcm::conv_shape(L, 16 / (int)bcm::dtype_size(dtype));
+  const int64_t blocks = (D + c.R - 1) / c.R * c.nseg;
+  if (blocks > INT32_MAX) return bcm::set_error(BCM_EINVAL, "%s: too many rows", fn);
+  const dim3 grid((unsigned)blocks, (unsigned)std::min<int64_t>(B, 65535));
   bcm::dispatch_dtype(dtype, [&](auto tag) {
     using T = decltype(tag);
-    auto go = [&](auto s_, auto v_) {
-      constexpr bool S = decltype(s_)::value, V = decltype(v_)::value;
+    auto go = [&](auto s_) {
+      constexpr bool S = decltype(s_)::value;
       if (K == 4)
-        hipLaunchKernelGGL((bcm::k_conv_fwd<T, S, V, 4>), grid, dim3(256), 0, bcm::hs(stream),
-                           static_cast<const T*>(x), weight, bias, static_cast<T*>(out), rows, (int)D, L, K, chunks);
+        hipLaunchKernelGGL((bcm::k_conv_fwd<T, S, 4>), grid, dim3(256), 0, bcm::hs(stream), static_cast<const T*>(x),
+                           weight, bias, static_cast<T*>(out), (int)B, (int)D, L, K, c.lg, (int)c.nseg);
       else
-        hipLaunchKernelGGL((bcm::k_conv_fwd<T, S, V, 8>), grid, dim3(256), 0, bcm::hs(stream),
-                           static_cast<const T*>(x), weight, bias, static_cast<T*>(out), rows, (int)D, L, K, chunks);
+        hipLaunchKernelGGL((bcm::k_conv_fwd<T, S, 8>), grid, dim3(256), 0, bcm::hs(stream), static_cast<const T*>(x),
+                           weight, bias, static_cast<T*>(out), (int)B, (int)D, L, K, c.lg, (int)c.nseg);
     };
-    if (silu) {
-      if (vec) go(std::true_type{}, std::true_type{});
-      else go(std::true_type{}, std::false_type{});
-    } else {
-      if (vec) go(std::false_type{}, std::true_type{});
-      else go(std::false_type{}, std::false_type{});
-    }
+    if (silu) go(std::true_type{});
+    else go(std::false_type{});
   });
   return bcm::check_launch(fn);
 }
 
 int64_t bcm_causal_conv1d_bwd_workspace_bytes(int64_t B, int64_t D, int64_t L, int K) {
-  (void)L;
-  if (B < 1 || D < 1 || K < 1 || K > bcm::kConvMaxK) return 0;
-  const int P = bcm::conv_split(B, D);
+  if (B < 1 || D < 1 || L < 1 || K < 1 || K > bcm::kConvMaxK) return 0;
+  const int P = bcm::conv_split(B, D, L);
   return P > 1 ? 4 * (int64_t)P * D * (K + 1) : 0;
 }
 
@@ -454,31 +502,27 @@ int bcm_causal_conv1d_bwd(const void* x, int dtype, const float* weight, const f
   if (rc) return rc;
   if (!weight || !dweight) return bcm::set_error(BCM_EINVAL, "%s: null pointer", fn);
   if (B > 0 && L > 0 && (!x || !dout || !dx)) return bcm::set_error(BCM_EINVAL, "%s: null pointer", fn);
-  int P = B > 0 ? bcm::conv_split(B, D) : 1;
+  int P = B > 0 && L > 0 ? bcm::conv_split(B, D, L) : 1;
   if (P > 1 && (!workspace || workspace_bytes < 4 * (int64_t)P * D * (K + 1))) P = 1;  // no room: one group
-  const bool vec = L % 4 == 0 && bcm::aligned16(x) && bcm::aligned16(dout) && bcm::aligned16(dx);
+  const bcm::ConvShape c = bcm::conv_shape(L, bcm::kConvS);
+  const int64_t units = L > 0 ? bcm::conv_units(B, L) : 0;
   float* part = static_cast<float*>(workspace);
   bcm::dispatch_dtype(dtype, [&](auto tag) {
     using T = decltype(tag);
-    auto go = [&](auto s_, auto v_) {
-      constexpr bool S = decltype(s_)::value, V = decltype(v_)::value;
+    auto go = [&](auto s_) {
+      constexpr bool S = decltype(s_)::value;
       const dim3 grid((unsigned)D, (unsigned)P);
       if (K == 4)
-        hipLaunchKernelGGL((bcm::k_conv_bwd<T, S, V, 4>), grid, dim3(256), 0, bcm::hs(stream),
-                           static_cast<const T*>(x), weight, bias, static_cast<const T*>(dout), static_cast<T*>(dx),
-                           dweight, dbias, part, (int)B, (int)D, L, K);
+        hipLaunchKernelGGL((bcm::k_conv_bwd<T, S, 4>), grid, dim3(256), 0, bcm::hs(stream), static_cast<const T*>(x),
+                           weight, bias, static_cast<const T*>(dout), static_cast<T*>(dx), dweight, dbias, part, (int)B,
+                           (int)D, L, K, c.lg, (int)c.nseg, units);
       else
-        hipLaunchKernelGGL((bcm::k_conv_bwd<T, S, V, 8>), grid, dim3(256), 0, bcm::hs(stream),
-                           static_cast<const T*>(x), weight, bias, static_cast<const T*>(dout), static_cast<T*>(dx),
-                           dweight, dbias, part, (int)B, (int)D, L, K);
+        hipLaunchKernelGGL((bcm::k_conv_bwd<T, S, 8>), grid, dim3(256), 0, bcm::hs(stream), static_cast<const T*>(x),
+                           weight, bias, static_cast<const T*>(dout), static_cast<T*>(dx), dweight, dbias, part, (int)B,
+                           (int)D, L, K, c.lg, (int)c.nseg, units);
     };
-    if (silu) {
-      if (vec) go(std::true_type{}, std::true_type{});
-      else go(std::true_type{}, std::false_type{});
-    } else {
-      if (vec) go(std::false_type{}, std::true_type{});
-      else go(std::false_type{}, std::false_type{});
-    }
+    if (silu) go(std::true_type{});
+    else go(std::false_type{});
   });
   rc = bcm::check_launch(fn);
   if (rc || P == 1) return rc;
