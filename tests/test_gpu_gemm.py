@@ -140,3 +140,16 @@ def test_gemm_leaves_other_products_to_torch(cuda_device):
         assert pj._kernel_form(f, f) is None
     for x, y in ((f.t(), f.t()), (f[:, ::2], f[:8]), (f[:1].expand(16, 16), f)):
         assert torch.allclose(pj.mm(x, y), x @ y)
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_gemm_errors_do_not_add_up(cuda_device, form):
+    """The errors of many results have no common direction: their mean over
+    n = 4096 x 256 results stays within 8 / sqrt(n) of their size (a rounding
+    in one direction leaves it near a twentieth of it)."""
+    x, y = _operands(4096, 256, 256, form, cuda_device, seed=6)
+    err = pj.mm(x, y).double() - x.double() @ y.double()
+    rms = float(err.pow(2).mean().sqrt())
+    assert abs(float(err.mean())) <= 8.0 * rms / (4096 * 256) ** 0.5
+    for dim, n in ((0, 4096), (1, 256)):  # and along either side
+        assert float(err.sum(dim).pow(2).mean().sqrt()) <= 2.0 * rms * n ** 0.5
