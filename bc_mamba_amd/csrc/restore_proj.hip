@@ -9,27 +9,29 @@
 // z[b, t, :], dz = dOut W, and dy[e] = sum of dz over the steps event e owns
 // (restore_dense_bwd_kernel.cuh:42-112).
 //
-// MI355X design: z [B, L, D] and dz never exist in HBM. The products run on
-// the matrix cores at their fp32 rate (v_mfma_f32_32x32x2_f32), on 64 x 64
-// output tiles of 4 waves (32 x 32 each). The contraction index of MFMA step
+// MI355X design: z [B, L, D] and dz never exist in HBM. The forward's and dW's
+// products run on the matrix cores at their fp32 rate (v_mfma_f32_32x32x2_f32),
+// on 64 x 64 output tiles of 4 waves (32 x 32 each). The contraction index of MFMA step
 // s pairs the two lane halves h as k = 16 h + s, so each lane's operand run
 // is 16 consecutive elements of one row (or of one channel's steps).
 //  - forward: per (b, 64-step tile j, 64 output columns), z is generated 32
 //    channels at a time into LDS from the event index (one tile-mask
 //    popcount and one gather per element, no search), double-buffered
 //    against the MFMAs; W fragments come from L2.
-//  - dy: the dz tile [64 steps x 64 channels] = dOut tile W[:, channels] is
-//    staged once in LDS; one wave then runs the restore backward's sweep
-//    over it (runs closed inside the tile go to dy; head, tail and last
-//    event to the fix-up arrays) and the restore backward's fix-up pass
-//    closes the runs that cross tiles. No atomics.
+//  - dy: the dz tile [128 steps x 128 channels] = dOut tile W[:, channels] is
+//    one tile of the split fp16 product (gemm_tile.hpp), staged once in
+//    LDS, where each thread runs the restore backward's sweep over one
+//    channel of one 64-step tile (runs closed inside the tile go to dy; head,
+//    tail and last event to the fix-up arrays); the restore backward's fix-up
+//    pass closes the runs that cross tiles. No atomics.
 //  - dW: per (64 rows of W, 64 channels, one sequence segment of up to
 //    1024 steps) a partial dOut^T z, with z generated per lane from the
 //    event index (16 consecutive steps of one channel per MFMA operand run),
 //    then a fixed-order sum of the partials (deterministic).
-// fp32 throughout: the MFMA products are exact and accumulate in fp32, as
-// the reference's fp32 GEMM does (in another order).
-#include "bcm_common.hpp"
+// fp32 accuracy throughout, as the reference's fp32 GEMM (in another order).
+#include "gemm_tile.hpp"
+
+#include <cstddef>
 
 namespace bcm {
 
@@ -38,7 +40,6 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kPT = 64;          // output tile edge
 constexpr int kKC = 32;          // contraction chunk (16 MFMA steps)
 constexpr int kRS = kKC + 4;     // LDS row stride of an operand chunk (16-byte rows, conflict-free 16-byte reads)
-constexpr int kDS = kPT + 1;     // LDS row stride of a dz tile
 constexpr int kSeg = 512;        // sequence steps per dW partial (1600 items at a config-4 layer)
 static_assert(kSeg % 64 == 0, "a dW segment starts a 64-step tile");
 
@@ -164,122 +165,117 @@ __global__ __launch_bounds__(256) void k_restore_proj_fwd(const float* __restric
 }
 
 // ------------------------------------------------------------- dy (dz pass)
-// Item (b, j, db): dz rows t0 .. t0 + 63, channels d0 = 64 db .. + 63. Per
-// 32-row chunk of W: the dOut tile columns [step][k] from coalesced row
-// loads, and W [k][channel] transposed into [channel][k] on its way to LDS,
-// so both MFMA operand runs are 16-byte LDS reads (double-buffered, one
-// barrier per chunk).
-__global__ __launch_bounds__(256) void k_restore_proj_dy(const float* __restrict__ dout, int64_t n_events,
-                                                         const uint32_t* __restrict__ bitmask, int64_t Wd,
-                                                         int64_t mrd, const int32_t* __restrict__ tile_start,
-                                                         int nT, int dim, int L, int64_t n_rows,
-                                                         const float* __restrict__ weight, int dm, int nDB,
-                                                         float* __restrict__ dy, float* __restrict__ head,
-                                                         float* __restrict__ tail, int32_t* __restrict__ tend) {
-  __shared__ float4 s_ab[2 * 2 * kPT * kRS / 4];
-  float* sA = reinterpret_cast<float*>(s_ab);  // [2][64][kRS]: dOut chunk [step][k]
-  float* sB = sA + 2 * kPT * kRS;              // [2][64][kRS]: W chunk [channel][k]
+// Item (b, jj, db): dz rows t0 = 128 jj .. t0 + 127 (two 64-step tiles),
+// channels d0 = 128 db .. + 127, as one tile of the split fp16 product
+// (gemm_tile.hpp: dOut rows against W's columns). The dz tile then goes to LDS
+// over the operand stages, and each thread runs the restore backward's sweep
+// over one channel of one 64-step tile: runs closed inside the tile go to dy,
+// the rest to the fix-up arrays. 51 200 tokens, d_model 256, d_inner 512:
+// 84 us, against 140-145 us on the fp32 matrix cores (64-channel items, two of
+// four waves sweeping).
+constexpr int kDyT = 128;            // dz rows (steps) per item
+constexpr int kDyS = kGT + 1;        // LDS row stride of the dz tile
+static_assert(sizeof(float) * kDyT * kDyS <= offsetof(GemmLds, exp), "the dz tile leaves the scale exponents alone");
+
+template <bool WHOLE>
+__global__ __launch_bounds__(256, 2) void k_restore_proj_dy(const float* __restrict__ dout, int64_t n_events,
+                                                            const uint32_t* __restrict__ bitmask, int64_t Wd,
+                                                            int64_t mrd, const int32_t* __restrict__ tile_start,
+                                                            int nT, int dim, int L, int64_t n_rows,
+                                                            const float* __restrict__ weight, int dm, int nDB,
+                                                            float* __restrict__ dy, float* __restrict__ head,
+                                                            float* __restrict__ tail, int32_t* __restrict__ tend) {
+  __shared__ GemmLds s;
   const int item = xcd_block(blockIdx.x, gridDim.x);
+  const int nJJ = (nT + 1) / 2;
   const int db = item % nDB, bj = item / nDB;
-  const int j = bj % nT, b = bj / nT;
-  const int t0 = j * kTile, d0 = db * kPT;
-  const int tid = threadIdx.x, lane = lane_id();
+  const int jj = bj % nJJ, b = bj / nJJ;
+  const int t0 = jj * kDyT, d0 = db * kGT;
+  const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int rb = 32 * (w & 1), cb = 32 * (w >> 1);
-  const int li = lane & 31, h = lane >> 5;
-  const int64_t gbase = ((int64_t)b * L + t0) * dm;
-  const __amdgpu_buffer_rsrc_t rg = buf_rsrc(dout + gbase, ((int64_t)(L - t0) * dm) * 4);
-  const __amdgpu_buffer_rsrc_t rw = buf_rsrc(weight, (int64_t)dm * dim * 4);
-  // dOut: step (tid >> 3) + 32 i, columns 4 (tid & 7) .. + 3 of the chunk;
-  // W: row (tid >> 6) + 4 i of the chunk, channel tid & 63
-  const int ac = 4 * (tid & 7), ar = tid >> 3, bc = tid & 63, br = tid >> 6;
-  float4 av[2];
-  float bv[8];
-  auto load = [&](int c) {
-    const int k = c * kKC + ac;
+  const float* g = dout + ((int64_t)b * L + t0) * dm;
+  gf16v acc[2][2] = {};
+  gemm_tile<true, false, WHOLE>(g, L - t0, dm, weight, dim, dim, dm, 0, d0, 0, dm, s, acc);  // rows past L are 0
+  float* sD = reinterpret_cast<float*>(&s.sm[0][0]);
+  const int col = gemm_col(w), eb0 = s.exp[gemm_slot_b(w, 0)], eb1 = s.exp[gemm_slot_b(w, 1)];
+  const bool inf = s.inf != 0;  // kept across the tile's stores (they end below it)
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int row = ar + 32 * i;
-      float v[4];
+  for (int ta = 0; ta < 2; ++ta)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        v[e] = buf_load<float>(rg, (t0 + row < L && k + e < dm) ? (uint32_t)(row * dm + k + e) * 4u : kBufOOB);
-      av[i] = make_float4(v[0], v[1], v[2], v[3]);
+    for (int r = 0; r < 16; ++r) {
+      const int row = gemm_row(w, ta, r), ea = s.exp[gemm_slot_a(w, ta, r)];
+      sD[row * kDyS + col] = gemm_value(acc[ta][0][r], ta, 0, ea + eb0);
+      sD[row * kDyS + col + 1] = gemm_value(acc[ta][1][r], ta, 1, ea + eb1);
     }
-    const int d = d0 + bc;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int kr = c * kKC + br + 4 * i;
-      bv[i] = buf_load<float>(rw, (kr < dm && d < dim) ? (uint32_t)(kr * dim + d) * 4u : kBufOOB);
+  __syncthreads();
+  if (__builtin_expect(inf, 0)) {  // an infinity in dOut or W: dz again with plain FMAs
+    for (int i = tid; i < kDyT * kGT; i += 256) {
+      const int t = i / kGT, d = d0 + i % kGT;
+      float v = 0.0f;
+      if (t0 + t < L && d < dim)
+        for (int k = 0; k < dm; ++k) v = fmaf(g[(int64_t)t * dm + k], weight[(int64_t)k * dim + d], v);
+      sD[t * kDyS + i % kGT] = v;
     }
-  };
-  const int nK = (dm + kKC - 1) / kKC;
-  f32x16 acc = {};
-  load(0);
-  for (int c = 0; c < nK; ++c) {
-    float* ab = sA + (c & 1) * kPT * kRS;
-    float* bb = sB + (c & 1) * kPT * kRS;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) *reinterpret_cast<float4*>(ab + (ar + 32 * i) * kRS + ac) = av[i];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) bb[bc * kRS + br + 4 * i] = bv[i];
     __syncthreads();
-    if (c + 1 < nK) load(c + 1);
-    const float4* aa = reinterpret_cast<const float4*>(ab + (rb + li) * kRS + 16 * h);
-    const float4* ba = reinterpret_cast<const float4*>(bb + (cb + li) * kRS + 16 * h);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float4 a = aa[v], bq = ba[v];
-      acc = mfma32(a.x, bq.x, acc);
-      acc = mfma32(a.y, bq.y, acc);
-      acc = mfma32(a.z, bq.z, acc);
-      acc = mfma32(a.w, bq.w, acc);
-    }
   }
-  // dz tile [64 steps][64 channels] in LDS (over the operand buffers)
-  __syncthreads();
-  float* sD = sA;
-  static_assert(4 * kPT * kRS >= kPT * kDS, "dz tile fits the operand buffers");
-#pragma unroll
-  for (int r = 0; r < 16; ++r) sD[(rb + acc_row(r, h)) * kDS + cb + li] = acc[r];
-  __syncthreads();
-  if (w != 0) return;
-  // one wave: lane = channel d0 + lane, the restore backward's sweep over
-  // the tile's 64 steps (rows past L hold 0 and have no event bits)
-  const int dd = d0 + lane;
+  // thread: channel d0 + tid % 128, tile 2 jj + tid / 128 (rows past L count
+  // as 0 and hold no event bits)
+  const int j = 2 * jj + (tid >> 7), cl = tid & (kGT - 1), dd = d0 + cl;
+  if (j >= nT) return;
   const bool ok = dd < dim;
   const int64_t ch = (int64_t)b * dim + (ok ? dd : dim - 1);
   const uint64_t m = ok ? tile_mask(bitmask + (ch / mrd) * Wd, j) : 0ull;
   const int32_t elo = tile_start[ch * (nT + 1) + j];
   const __amdgpu_buffer_rsrc_t rdy = buf_rsrc(dy, n_events * 4);
-  const int first = m ? __builtin_ctzll(m) : kTile;
-  uint32_t r = 0;  // events seen so far in the tile
-  float sum = 0.0f, hsum = 0.0f;
-  for (int s = 0; s < kTile; ++s) {
-    const float gv = sD[s * kDS + lane];
-    const uint32_t bit = (uint32_t)(m >> s) & 1u;
-    // the run of event elo + r - 1 closes here when r >= 1
-    buf_store_f32(rdy, (bit && r) ? (uint32_t)(elo + (int32_t)r - 1) * 4u : kBufOOB, sum);
-    r += bit;
-    sum = (bit ? 0.0f : sum) + gv;
-    hsum += s < first ? gv : 0.0f;
+  // The sweep: the sum up to here goes into row r of the channel's own column
+  // at every step (r events seen, rows up to the step are read by then), so
+  // when an event closes the run, row r holds it: row 0 the head, row i + 1
+  // the run of the tile's i-th event. From there the runs go to dy as the
+  // channel's events lie (stores of one value per channel and step would touch
+  // 64 lines each).
+  float* col_s = sD + (tid >> 7) * kTile * kDyS + cl;
+  const uint32_t mw[2] = {(uint32_t)m, (uint32_t)(m >> 32)};
+  uint32_t at = 0;  // byte offset of row r
+  float sum = 0.0f;
+#pragma unroll
+  for (int s0 = 0; s0 < kTile; s0 += 16) {
+    float gv[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) gv[i] = col_s[(s0 + i) * kDyS];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int32_t mk = __builtin_amdgcn_sbfe((int32_t)mw[s0 >> 5], (uint32_t)(s0 + i) & 31u, 1u);  // 0 / -1
+      *reinterpret_cast<float*>(reinterpret_cast<char*>(col_s) + at) = sum;
+      at += (uint32_t)mk & (uint32_t)(kDyS * 4);
+      sum = __uint_as_float(__float_as_uint(sum) & ~(uint32_t)mk) + gv[i];
+    }
   }
+  const int r = __builtin_popcountll(m);
   if (ok) {
     const int64_t o = (int64_t)j * n_rows + ch;
-    head[o] = hsum;
+    head[o] = r ? col_s[0] : sum;
     tail[o] = sum;
-    tend[o] = r ? elo + (int32_t)r : -1;
+    tend[o] = r ? elo + r : -1;
+  }
+  wave_sync();
+  // half a wave per channel: 32 of its closed runs at a time
+  const int hl = lane_id() & 31, hw = lane_id() >> 5;
+  const float* tile_s = sD + (tid >> 7) * kTile * kDyS + (cl & 64);
+  const int most = wave_max(r) - 1;
+  for (int r0 = 0; r0 < most; r0 += 32) {
+#pragma unroll 8
+    for (int c = 0; c < kWave; c += 2) {
+      const int n0 = __builtin_amdgcn_readlane(r, c), n1 = __builtin_amdgcn_readlane(r, c + 1);
+      const int x0 = __builtin_amdgcn_readlane(elo, c), x1 = __builtin_amdgcn_readlane(elo, c + 1);
+      const int n = (hw ? n1 : n0) - 1, i = r0 + hl;
+      const float v = tile_s[min(i + 1, kTile - 1) * kDyS + c + hw];
+      buf_store_f32(rdy, i < n ? (uint32_t)((hw ? x1 : x0) + i) * 4u : kBufOOB, v);
+    }
   }
 }
 
-// ------------------------------------------------- dy, LDS-DMA form
-// The dy product with both operands brought in by LDS DMA (gfx950's
-// global_load_lds_dwordx4: 16 bytes per lane straight into LDS, no register
-// staging), two stages in flight; for d_model % 32 == 0 and dim % 64 == 0
-// (the items then never straddle the contraction or channel ends).
-// Item (b, jj, db): dz rows t0 = 128 jj .. t0 + 127 (two 64-step tiles),
-// channels d0 = 64 db .. + 63. Wave w: steps 64 (w & 1) .. + 63 (two 32-row
-// MFMA blocks sharing one W fragment), channels 32 (w >> 1) .. + 31.
+// LDS DMA (gfx950's global_load_lds_dwordx4: 16 bytes per lane straight into
+// LDS, no register staging).
 typedef __attribute__((address_space(3))) void* lds_vptr;
 __device__ __forceinline__ uint32_t lds_off(const void* p) { return (uint32_t)(size_t)(lds_vptr)p; }
 // 16 bytes per lane from gptr into LDS at the wave-uniform byte offset off +
@@ -294,108 +290,7 @@ __device__ __forceinline__ void wait_vmcnt0() { asm volatile("s_waitcnt vmcnt(0)
 // the 8 row pairs rotate them, so 16 consecutive rows reading the same slot
 // hit 16 different bank groups
 __device__ __forceinline__ int qswz(int row) { return (row >> 1) & 7; }
-constexpr int kDyT = 128;  // dz rows (steps) per item of the DMA form
-
-__global__ __launch_bounds__(256) void k_restore_proj_dy_dma(const float* __restrict__ dout, int64_t n_events,
-                                                             const uint32_t* __restrict__ bitmask, int64_t Wd,
-                                                             int64_t mrd, const int32_t* __restrict__ tile_start,
-                                                             int nT, int dim, int L, int64_t n_rows,
-                                                             const float* __restrict__ weight, int dm, int nDB,
-                                                             float* __restrict__ dy, float* __restrict__ head,
-                                                             float* __restrict__ tail, int32_t* __restrict__ tend) {
-  extern __shared__ float4 s_dyn[];
-  float* sA = reinterpret_cast<float*>(s_dyn);  // [2][128][32]: dOut rows, slots swizzled
-  float* sB = sA + 2 * kDyT * kKC;              // [2][32][64]: W rows of the item's channels
-  const int item = xcd_block(blockIdx.x, gridDim.x);
-  const int nJJ = (nT + 1) / 2;
-  const int db = item % nDB, bj = item / nDB;
-  const int jj = bj % nJJ, b = bj / nJJ;
-  const int t0 = jj * kDyT, d0 = db * kPT;
-  const int tid = threadIdx.x, lane = lane_id();
-  const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int li = lane & 31, h = lane >> 5;
-  const int rb = 64 * (w & 1), cb = 32 * (w >> 1);
-  const float* gb = dout + (int64_t)b * L * dm;
-  auto issue = [&](int c, int st) {
-    // dOut: 16 wave loads of 8 rows each (4 per wave); rows past L read row
-    // L - 1 (their dz is not used)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int blk = 4 * w + i;
-      const int row = blk * 8 + (lane >> 3);
-      const int q = (lane & 7) ^ qswz(row);
-      const int t = min(t0 + row, L - 1);
-      lds_dma16(gb + (int64_t)t * dm + c * kKC + 4 * q, lds_off(sA + st * kDyT * kKC + blk * 256));
-    }
-    // W: 8 wave loads of 4 rows of 64 channels (2 per wave)
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int blk = 2 * w + i;
-      const int kr = blk * 4 + (lane >> 4);
-      lds_dma16(weight + (int64_t)(c * kKC + kr) * dim + d0 + 4 * (lane & 15),
-                lds_off(sB + st * kKC * kPT + blk * 256));
-    }
-  };
-  const int nK = dm / kKC;
-  f32x16 acc0 = {}, acc1 = {};
-  issue(0, 0);
-  for (int c = 0; c < nK; ++c) {
-    wait_vmcnt0();    // this wave's part of stage c has landed
-    __syncthreads();  // everyone's has, and every wave is done with stage c - 1
-    if (c + 1 < nK) issue(c + 1, (c + 1) & 1);
-    const float* ab = sA + (c & 1) * kDyT * kKC;
-    const float* bb = sB + (c & 1) * kKC * kPT;
-    const float4* a0 = reinterpret_cast<const float4*>(ab + (rb + li) * kKC);
-    const float4* a1 = reinterpret_cast<const float4*>(ab + (rb + 32 + li) * kKC);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float4 p0 = a0[(4 * h + v) ^ qswz(rb + li)], p1 = a1[(4 * h + v) ^ qswz(rb + 32 + li)];
-      const float* bk = bb + (16 * h + 4 * v) * kPT + cb + li;
-      acc0 = mfma32(p0.x, bk[0], acc0);
-      acc1 = mfma32(p1.x, bk[0], acc1);
-      acc0 = mfma32(p0.y, bk[kPT], acc0);
-      acc1 = mfma32(p1.y, bk[kPT], acc1);
-      acc0 = mfma32(p0.z, bk[2 * kPT], acc0);
-      acc1 = mfma32(p1.z, bk[2 * kPT], acc1);
-      acc0 = mfma32(p0.w, bk[3 * kPT], acc0);
-      acc1 = mfma32(p1.w, bk[3 * kPT], acc1);
-    }
-  }
-  // dz tile [128 steps][64 channels] in LDS over the operand stages
-  __syncthreads();
-  float* sD = sA;
-  static_assert(2 * kDyT * kKC + 2 * kKC * kPT >= kDyT * kDS, "dz tile fits the operand stages");
-#pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    sD[(rb + acc_row(r, h)) * kDS + cb + li] = acc0[r];
-    sD[(rb + 32 + acc_row(r, h)) * kDS + cb + li] = acc1[r];
-  }
-  __syncthreads();
-  // waves 0 and 1: the restore backward's sweep over tile 2 jj + w, lane =
-  // channel d0 + lane (rows past L count as 0 and hold no event bits)
-  const int j = 2 * jj + w;
-  if (w > 1 || j >= nT) return;
-  const int64_t ch = (int64_t)b * dim + d0 + lane;
-  const uint64_t m = tile_mask(bitmask + (ch / mrd) * Wd, j);
-  const int32_t elo = tile_start[ch * (nT + 1) + j];
-  const __amdgpu_buffer_rsrc_t rdy = buf_rsrc(dy, n_events * 4);
-  const int first = m ? __builtin_ctzll(m) : kTile;
-  const int steps = min(kTile, L - j * kTile);
-  uint32_t r = 0;
-  float sum = 0.0f, hsum = 0.0f;
-  for (int s = 0; s < kTile; ++s) {
-    const float gv = s < steps ? sD[(64 * w + s) * kDS + lane] : 0.0f;
-    const uint32_t bit = (uint32_t)(m >> s) & 1u;
-    buf_store_f32(rdy, (bit && r) ? (uint32_t)(elo + (int32_t)r - 1) * 4u : kBufOOB, sum);
-    r += bit;
-    sum = (bit ? 0.0f : sum) + gv;
-    hsum += s < first ? gv : 0.0f;
-  }
-  const int64_t o = (int64_t)j * n_rows + ch;
-  head[o] = hsum;
-  tail[o] = sum;
-  tend[o] = r ? elo + (int32_t)r : -1;
-}
+constexpr int kFwT = 128;  // out rows (steps) per item of the forward's DMA form
 
 // --------------------------------------------- forward, LDS-DMA form
 // The forward with W brought in by LDS DMA and z generated into LDS, for
@@ -416,13 +311,13 @@ __global__ __launch_bounds__(256) void k_restore_proj_fwd_dma(const float* __res
                                                               float* __restrict__ out) {
   extern __shared__ float4 s_dyn[];
   float* sZ = reinterpret_cast<float*>(s_dyn);                // [2][128][32]: z rows (steps)
-  float* sW = sZ + 2 * kDyT * kKC;                            // [2][64][32]: W rows (columns of out)
+  float* sW = sZ + 2 * kFwT * kKC;                            // [2][64][32]: W rows (columns of out)
   uint4* sIdx = reinterpret_cast<uint4*>(sW + 2 * kPT * kKC);  // [2][dim]: mask lo, hi, tsj, first
   const int item = xcd_block(blockIdx.x, gridDim.x);
   const int nJJ = (nT + 1) / 2;
   const int nb = item % nNB, bj = item / nNB;
   const int jj = bj % nJJ, b = bj / nJJ;
-  const int t0 = jj * kDyT, n0 = nb * kPT;
+  const int t0 = jj * kFwT, n0 = nb * kPT;
   const int tid = threadIdx.x, lane = lane_id();
   const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int li = lane & 31, h = lane >> 5;
@@ -462,7 +357,7 @@ __global__ __launch_bounds__(256) void k_restore_proj_fwd_dma(const float* __res
   gen(0);
   const int zrow = 64 * th + lane;
   for (int c = 0; c < nK; ++c) {
-    float* zb = sZ + (c & 1) * kDyT * kKC;
+    float* zb = sZ + (c & 1) * kFwT * kKC;
     float4* zrw = reinterpret_cast<float4*>(zb + zrow * kKC);
 #pragma unroll
     for (int qq = 0; qq < 4; ++qq)
@@ -808,7 +703,7 @@ int bcm_restore_proj_fwd(const float* y, int64_t n_events, const uint32_t* bitma
   // and 16-byte aligned W rows; its per-channel index words take 32 bytes
   // of LDS per channel, so wide layers (dim above ~3.5k on a 160 KB part)
   // take the register-staged form, which needs 16
-  const size_t lds_dma = (size_t)(2 * kDyT * kKC + 2 * kPT * kKC) * 4 + (size_t)dim * 32;
+  const size_t lds_dma = (size_t)(2 * kFwT * kKC + 2 * kPT * kKC) * 4 + (size_t)dim * 32;
   const bool dma = dim % kKC == 0 && d_model % kPT == 0 && (reinterpret_cast<uintptr_t>(weight) & 15) == 0 &&
                    (int64_t)lds_dma <= max_lds_bytes();
   if (dma) {
@@ -858,21 +753,16 @@ int bcm_restore_proj_bwd(const float* dout, const float* y, int64_t n_events, co
   int32_t* tend = reinterpret_cast<int32_t*>(tail + s.nT * n_rows);
   float* part = reinterpret_cast<float*>(tend + s.nT * n_rows);
   if (dy && n_events > 0) {
-    // the LDS-DMA form wants whole 32-row chunks of W, whole 64-channel
-    // blocks and 16-byte aligned rows
-    const bool dma = d_model % kKC == 0 && dim % kPT == 0 && (reinterpret_cast<uintptr_t>(dout) & 15) == 0 &&
-                     (reinterpret_cast<uintptr_t>(weight) & 15) == 0;
-    if (dma) {
-      const int64_t nJJ = (s.nT + 1) / 2;
-      const size_t lds = (size_t)(2 * kDyT * kKC + 2 * kKC * kPT) * 4;
-      hipLaunchKernelGGL(k_restore_proj_dy_dma, dim3((unsigned)(B * nJJ * s.nDB)), dim3(256), lds, st, dout,
-                         n_events, bitmask, s.W, mask_row_div, tile_start, (int)s.nT, (int)dim, (int)L, n_rows,
-                         weight, (int)d_model, (int)s.nDB, dy, head, tail, tend);
-    } else {
-      hipLaunchKernelGGL(k_restore_proj_dy, dim3((unsigned)(B * s.nT * s.nDB)), dim3(256), 0, st, dout, n_events,
-                         bitmask, s.W, mask_row_div, tile_start, (int)s.nT, (int)dim, (int)L, n_rows, weight,
-                         (int)d_model, (int)s.nDB, dy, head, tail, tend);
-    }
+    const int64_t nJJ = (s.nT + 1) / 2, nDB = (dim + kGT - 1) / kGT;
+    const dim3 grid((unsigned)(B * nJJ * nDB));
+    if (d_model % kGK == 0 && dim % 4 == 0)
+      hipLaunchKernelGGL(k_restore_proj_dy<true>, grid, dim3(256), 0, st, dout, n_events, bitmask, s.W, mask_row_div,
+                         tile_start, (int)s.nT, (int)dim, (int)L, n_rows, weight, (int)d_model, (int)nDB, dy, head,
+                         tail, tend);
+    else
+      hipLaunchKernelGGL(k_restore_proj_dy<false>, grid, dim3(256), 0, st, dout, n_events, bitmask, s.W, mask_row_div,
+                         tile_start, (int)s.nT, (int)dim, (int)L, n_rows, weight, (int)d_model, (int)nDB, dy, head,
+                         tail, tend);
     if ((rc = check_launch(fn))) return rc;
     if ((rc = restore_bwd_fix(s.nT, n_rows, head, tail, tend, dy, n_events, st, fn))) return rc;
   }
