@@ -117,6 +117,8 @@ SIGNATURES = {
     "bcm_gemm_f32_workspace_bytes": (c_i64, [c_i64, c_i64, c_i64]),
     "bcm_gemm_f32": (c_i32, [c_p, c_i32, c_i64, c_p, c_i32, c_i64, c_p, c_i64, c_i64, c_i64, c_p, c_i64, c_p, c_i64,
                              c_p]),
+    "bcm_block_params_fwd": (c_i32, [c_p, c_p, c_p, c_p, c_i64, c_i64, c_f32, c_p, c_p, c_p, c_p, c_p, c_p]),
+    "bcm_block_params_bwd": (c_i32, [c_p, c_p, c_p, c_i64, c_i64] + [c_p] * 10),
 }
 
 RESTORE_BWD_NOALLOC_MAX_TILES = 699040  # BCM_RESTORE_BWD_NOALLOC_MAX_TILES of the header

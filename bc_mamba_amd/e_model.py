@@ -310,6 +310,44 @@ class TwoLevelDelta(nn.Module):
         return F.softplus(self.a0) + self.eps, F.softplus(self.a1) + self.eps
 
 
+class _BlockParamsFn(torch.autograd.Function):
+    """The scan parameters (dt_idle, dt_active, A, W_B, W_C) from the block's
+    learned ones (TwoLevelDelta.a0 and a1, A_log, W_BC) as one kernel each
+    way (bcm_block_params_fwd / _bwd)."""
+
+    @staticmethod
+    def forward(ctx, a0, a1, A_log, W_BC, eps: float):
+        (D, N), dev = A_log.shape, A_log.device
+        dt_idle, dt_active = torch.empty_like(a0), torch.empty_like(a1)
+        A, W_B, W_C = (torch.empty_like(A_log) for _ in range(3))
+        with torch.cuda.device(dev):
+            _nat.call("bcm_block_params_fwd", a0.data_ptr(), a1.data_ptr(), A_log.data_ptr(), W_BC.data_ptr(), D, N,
+                      eps, dt_idle.data_ptr(), dt_active.data_ptr(), A.data_ptr(), W_B.data_ptr(), W_C.data_ptr(),
+                      _nat.stream_of(a0))
+        ctx.save_for_backward(a0, a1, A)
+        ctx.set_materialize_grads(False)
+        return dt_idle, dt_active, A, W_B, W_C
+
+    @staticmethod
+    def backward(ctx, *grads):
+        a0, a1, A = ctx.saved_tensors
+        D, N = A.shape
+        if torch.is_grad_enabled():  # a graph of the gradients is asked for: torch's operations
+            gi, ga, gA, gB, gC = (A.new_zeros(s) if g is None else g
+                                  for g, s in zip(grads, (D, D, (D, N), (D, N), (D, N))))
+            # softplus' derivative, 1 past its threshold
+            s0, s1 = (torch.where(a > 20.0, torch.ones_like(a), torch.sigmoid(a)) for a in (a0, a1))
+            return gi * s0, ga * s1, gA * A, torch.cat((gB, gC), 1), None
+        grads = [g.contiguous() if g is not None else None for g in grads]
+        da0, da1, dA_log = torch.empty_like(a0), torch.empty_like(a1), torch.empty_like(A)
+        dW_BC = torch.empty((D, 2 * N), dtype=A.dtype, device=A.device)
+        with torch.cuda.device(A.device):
+            _nat.call("bcm_block_params_bwd", a0.data_ptr(), a1.data_ptr(), A.data_ptr(), D, N,
+                      *(_nat.ptr(g) for g in grads), da0.data_ptr(), da1.data_ptr(), dA_log.data_ptr(),
+                      dW_BC.data_ptr(), _nat.stream_of(A))
+        return da0, da1, dA_log, dW_BC, None
+
+
 class _SpikeBitsFn(torch.autograd.Function):
     """The "ste" spike s = (p >= thr) + p - p with its identity gradient, as
     one kernel that also emits the event bitmask of the transposed spikes
@@ -470,6 +508,22 @@ class Mamba(nn.Module):
                 and seqlen * self.d_model * 4 < 2 ** 31 and self.d_model * self.d_inner * 4 < 2 ** 31
                 and (self.fused_out_proj != "mfma" or self.d_inner <= 7936))
 
+    def _scan_params(self):
+        """dt_idle, dt_active, A, W_B, W_C. The fused path takes them from one
+        kernel where the learned parameters are its own, contiguous fp32 on
+        the GPU (and nothing traces or casts the torch form)."""
+        g = self.delta_gen
+        ps = (g.a0, g.a1, self.A_log, self.W_BC) if type(g) is TwoLevelDelta else ()
+        if (self.fused_event_path and ps and not torch.compiler.is_compiling() and "levels" not in vars(g)
+                and all(type(q) in (torch.Tensor, nn.Parameter) and q.is_cuda and q.dtype == torch.float32
+                        and q.is_contiguous() and q.device == ps[0].device for q in ps)
+                and g.a0.shape == g.a1.shape == (self.d_inner,) and self.A_log.shape == (self.d_inner, self.d_state)
+                and self.W_BC.shape == (self.d_inner, 2 * self.d_state)):
+            return _BlockParamsFn.apply(*ps, float(g.eps))
+        dt_idle, dt_active = g.levels()
+        return (dt_idle, dt_active, -torch.exp(self.A_log), self.W_BC[:, :self.d_state].contiguous(),
+                self.W_BC[:, self.d_state:].contiguous())
+
     def forward(self, hidden_states, inference_params=None):
         if inference_params is not None:
             raise RuntimeError("Mamba: the decode / inference-cache path is not part of the event-path build")
@@ -485,10 +539,7 @@ class Mamba(nn.Module):
         if not conv_ev:
             x = self._conv(x, seqlen).contiguous()
 
-        dt_idle, dt_active = self.delta_gen.levels()
-        A = -torch.exp(self.A_log)
-        W_B = self.W_BC[:, :self.d_state].contiguous()
-        W_C = self.W_BC[:, self.d_state:].contiguous()
+        dt_idle, dt_active, A, W_B, W_C = self._scan_params()
         n_ch = batch * self.d_inner
 
         if self.fused_event_path:

@@ -553,6 +553,20 @@ int bcm_gemm_f32(const float* a, int a_k_contiguous, int64_t lda, const float* b
                  int64_t N, int64_t K, float* c, int64_t ldc, void* workspace,
                  int64_t workspace_bytes, bcm_stream_t stream);
 
+/* ---- (5) the block's scan parameters ------------------------------------ */
+/* dt_idle, dt_active [D] = softplus(a0), softplus(a1) + eps (TwoLevelDelta,
+ * e_model.py:210-230), A [D, N] = -exp(a_log), W_B and W_C [D, N] the halves
+ * of w_bc's rows [D, 2 N] (e_model.py:455-470); all fp32. The backward takes
+ * the gradients of the five (NULL: zero) and A as the forward gave it. */
+int bcm_block_params_fwd(const float* a0, const float* a1, const float* a_log,
+                         const float* w_bc, int64_t D, int64_t N, float eps,
+                         float* dt_idle, float* dt_active, float* A, float* W_B,
+                         float* W_C, bcm_stream_t stream);
+int bcm_block_params_bwd(const float* a0, const float* a1, const float* A, int64_t D,
+                         int64_t N, const float* g_idle, const float* g_active,
+                         const float* gA, const float* gB, const float* gC, float* da0,
+                         float* da1, float* da_log, float* dw_bc, bcm_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
