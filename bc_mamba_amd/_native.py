@@ -124,6 +124,7 @@ SIGNATURES = {
 RESTORE_BWD_NOALLOC_MAX_TILES = 699040  # BCM_RESTORE_BWD_NOALLOC_MAX_TILES of the header
 
 _lib = None
+_fns = {}  # name -> bound function
 
 
 def lib():
@@ -139,6 +140,7 @@ def lib():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
+            _fns[name] = fn
         if handle.bcm_abi_version() != ABI_VERSION:
             raise RuntimeError("bc_mamba_amd: ABI version mismatch")
         _lib = handle
@@ -147,13 +149,36 @@ def lib():
 
 def call(name, *args):
     """Call a C-ABI entry point and turn a non-zero status into RuntimeError."""
-    rc = getattr(lib(), name)(*args)
+    fn = _fns.get(name) if _lib is not None else getattr(lib(), name)
+    rc = fn(*args)
     if rc != 0:
         raise RuntimeError(lib().bcm_last_error().decode())
 
 
 def ptr(t):
-    return None if t is None else c_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+class _Here:
+    __slots__ = ()
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE_GUARD = _Here()
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
+def on_device(dev):
+    """torch.cuda.device(dev), or nothing to enter and leave where dev is the
+    current device already."""
+    if _current_device is not None and dev.index is not None and _current_device() == dev.index:
+        return _HERE_GUARD
+    return torch.cuda.device(dev)
 
 
 def dtype_code(dtype):

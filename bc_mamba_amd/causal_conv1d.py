@@ -20,11 +20,6 @@ except ImportError:  # imported with this directory on sys.path
 __all__ = ["causal_conv1d_fn", "CausalConv1dFn", "conv1d_bwd_events"]
 
 
-def _check(cond, msg):
-    if not cond:
-        raise RuntimeError(msg)
-
-
 class CausalConv1dFn(torch.autograd.Function):
     """out = act(bias + sum_k w[:, k] x[..., t-(K-1)+k]) with x = 0 before t=0;
     backward gives dx, dweight [D, K] and dbias (fp32 weights)."""
@@ -36,7 +31,7 @@ class CausalConv1dFn(torch.autograd.Function):
         b = bias.contiguous().float() if bias is not None else None
         B, D, L = x.shape
         out = torch.empty_like(x)
-        with torch.cuda.device(x.device):
+        with _nat.on_device(x.device):
             _nat.call("bcm_causal_conv1d_fwd", x.data_ptr(), _nat.dtype_code(x.dtype), w.data_ptr(),
                       b.data_ptr() if b is not None else None, B, D, L, int(w.size(1)), int(silu), out.data_ptr(),
                       _nat.stream_of(x))
@@ -53,7 +48,7 @@ class CausalConv1dFn(torch.autograd.Function):
         dw = torch.empty_like(w)
         db = torch.empty(D, dtype=torch.float32, device=x.device) if ctx.has_bias else None
         K = int(w.size(1))
-        with torch.cuda.device(x.device):
+        with _nat.on_device(x.device):
             nbytes = int(_nat.lib().bcm_causal_conv1d_bwd_workspace_bytes(B, D, L, K))
             ws = torch.empty(max(nbytes, 4) // 4, dtype=torch.float32, device=x.device) if nbytes else None
             _nat.call("bcm_causal_conv1d_bwd", x.data_ptr(), _nat.dtype_code(x.dtype), w.data_ptr(),
@@ -73,12 +68,13 @@ def conv1d_bwd_events(x, weight, bias, silu, du, event_index):
     bitmask, tile_start, mrd = event_index
     w = weight.detach().float().contiguous()
     b = bias.detach().float().contiguous() if bias is not None else None
-    _check(du.dtype == x.dtype and du.is_contiguous(), "conv1d_bwd_events: du must be contiguous, x's dtype")
+    if not (du.dtype == x.dtype and du.is_contiguous()):
+        raise RuntimeError("conv1d_bwd_events: du must be contiguous, x's dtype")
     dx = torch.empty_strided(x.shape, x.stride(), dtype=x.dtype, device=x.device)
     dw = torch.empty_like(w)
     db = torch.empty(D, dtype=torch.float32, device=x.device) if bias is not None else None
     K = int(w.size(1))
-    with torch.cuda.device(x.device):
+    with _nat.on_device(x.device):
         nbytes = int(_nat.lib().bcm_causal_conv1d_bwd_events_workspace_bytes(B, D, K))
         ws = torch.empty(max(nbytes, 4) // 4, dtype=torch.float32, device=x.device)
         _nat.call("bcm_causal_conv1d_bwd_events", x.data_ptr(), _nat.dtype_code(x.dtype), x.stride(0), x.stride(1),
@@ -93,13 +89,20 @@ def causal_conv1d_fn(x, weight, bias=None, seq_idx=None, initial_states=None, re
                      final_states_out=None, activation=None):
     """x [B, D, L] (fp32/fp16/bf16, CUDA), weight [D, K] (K <= 8), bias [D]."""
     fn = "causal_conv1d_fn"
-    _check(activation in (None, "silu", "swish"), f"{fn}: activation must be None, silu or swish")
-    _check(seq_idx is None and initial_states is None and not return_final_states and final_states_out is None,
-           f"{fn}: seq_idx / initial_states / final states are not supported by the MI355X build")
-    _check(x.is_cuda and weight.is_cuda and (bias is None or bias.is_cuda), f"{fn}: tensors must be on the GPU")
-    _check(x.dim() == 3, f"{fn}: x must be [batch, dim, seqlen]")
-    _check(weight.dim() == 2 and weight.size(0) == x.size(1), f"{fn}: weight must be [dim, width]")
-    _check(1 <= weight.size(1) <= 8, f"{fn}: width must be in [1, 8]")
-    _check(bias is None or tuple(bias.shape) == (x.size(1),), f"{fn}: bias must be [dim]")
-    _check(x.dtype in (torch.float32, torch.float16, torch.bfloat16), f"{fn}: x must be fp32/fp16/bf16")
+    if activation not in (None, "silu", "swish"):
+        raise RuntimeError(f"{fn}: activation must be None, silu or swish")
+    if not (seq_idx is None and initial_states is None and not return_final_states and final_states_out is None):
+        raise RuntimeError(f"{fn}: seq_idx / initial_states / final states are not supported by the MI355X build")
+    if not (x.is_cuda and weight.is_cuda and (bias is None or bias.is_cuda)):
+        raise RuntimeError(f"{fn}: tensors must be on the GPU")
+    if x.dim() != 3:
+        raise RuntimeError(f"{fn}: x must be [batch, dim, seqlen]")
+    if not (weight.dim() == 2 and weight.size(0) == x.size(1)):
+        raise RuntimeError(f"{fn}: weight must be [dim, width]")
+    if not (1 <= weight.size(1) <= 8):
+        raise RuntimeError(f"{fn}: width must be in [1, 8]")
+    if not (bias is None or tuple(bias.shape) == (x.size(1),)):
+        raise RuntimeError(f"{fn}: bias must be [dim]")
+    if x.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+        raise RuntimeError(f"{fn}: x must be fp32/fp16/bf16")
     return CausalConv1dFn.apply(x, weight, bias, activation in ("silu", "swish"))

@@ -320,7 +320,7 @@ class _BlockParamsFn(torch.autograd.Function):
         (D, N), dev = A_log.shape, A_log.device
         dt_idle, dt_active = torch.empty_like(a0), torch.empty_like(a1)
         A, W_B, W_C = (torch.empty_like(A_log) for _ in range(3))
-        with torch.cuda.device(dev):
+        with _nat.on_device(dev):
             _nat.call("bcm_block_params_fwd", a0.data_ptr(), a1.data_ptr(), A_log.data_ptr(), W_BC.data_ptr(), D, N,
                       eps, dt_idle.data_ptr(), dt_active.data_ptr(), A.data_ptr(), W_B.data_ptr(), W_C.data_ptr(),
                       _nat.stream_of(a0))
@@ -341,7 +341,7 @@ class _BlockParamsFn(torch.autograd.Function):
         grads = [g.contiguous() if g is not None else None for g in grads]
         da0, da1, dA_log = torch.empty_like(a0), torch.empty_like(a1), torch.empty_like(A)
         dW_BC = torch.empty((D, 2 * N), dtype=A.dtype, device=A.device)
-        with torch.cuda.device(A.device):
+        with _nat.on_device(A.device):
             _nat.call("bcm_block_params_bwd", a0.data_ptr(), a1.data_ptr(), A.data_ptr(), D, N,
                       *(_nat.ptr(g) for g in grads), da0.data_ptr(), da1.data_ptr(), dA_log.data_ptr(),
                       dW_BC.data_ptr(), _nat.stream_of(A))
@@ -483,7 +483,7 @@ class Mamba(nn.Module):
         it as the HIP causal conv (causal_conv1d_fn, the reference's fast
         path); the reference composition keeps nn.Conv1d, its fallback."""
         if self.fused_event_path:
-            return causal_conv1d_fn(x, self.conv1d.weight[:, 0, :], self.conv1d.bias, activation="silu")
+            return causal_conv1d_fn(x, self.conv1d.weight.squeeze(1), self.conv1d.bias, activation="silu")
         return self.act(self.conv1d(x)[..., :seqlen])
 
     def _conv_at_events_ok(self, x):
@@ -532,7 +532,7 @@ class Mamba(nn.Module):
             xw = projections.proj_tokens_last(self.in_proj.weight, hidden_states.reshape(batch * seqlen, dim))
         else:
             xw = self.in_proj.weight @ rearrange(hidden_states, "b l d -> d (b l)")
-        x = rearrange(xw, "d (b l) -> b d l", l=seqlen)
+        x = xw.reshape(-1, batch, seqlen).transpose(0, 1)  # "d (b l) -> b d l"
         if self.in_proj.bias is not None:
             x = x + rearrange(self.in_proj.bias.to(dtype=x.dtype), "d -> d 1")
         conv_ev = self._conv_at_events_ok(x)
@@ -548,7 +548,7 @@ class Mamba(nn.Module):
             bits = _event_bits_of(hidden_states, self.threshold)
             base_input = None if bits is not None else \
                 rearrange(hidden_states.detach(), "b l d -> b d l").contiguous()
-            w_conv, b_conv = self.conv1d.weight[:, 0, :], self.conv1d.bias
+            w_conv, b_conv = self.conv1d.weight.squeeze(1), self.conv1d.bias
             with cuda_stage("routing_index_extraction"):
                 _ch, time_steps, k_flat, cu_seqlens, max_seqlen, x_ev, event_index = \
                     _ee_cuda.extract_events_indexed(base_input, self.threshold, self.expand, x.detach(),

@@ -24,11 +24,6 @@ __all__ = ["extract_events", "extract_base_events", "expand_base_events",
 _I32 = torch.int32
 
 
-def _check(cond, msg):
-    if not cond:
-        raise RuntimeError(msg)
-
-
 def _empty_i32(n, dev):
     return torch.empty(n, dtype=_I32, device=dev)
 
@@ -82,14 +77,17 @@ def extract_base_events(base_input, threshold):
     cu_seqlens: restore_dense_fwd / _bwd, gather_events_bwd and the scan
     read them instead of recomputing them while those tensors are unchanged
     (bc_mamba_amd._provenance)."""
-    _check(base_input.is_cuda, "base_input must be CUDA")
-    _check(base_input.is_contiguous(), "base_input must be contiguous")
-    _check(base_input.dim() == 3, "base_input must be 3-D [B, d_model, L]")
-    _check(base_input.dtype in (torch.float32, torch.float16, torch.bfloat16),
-           "base_input must be fp32, fp16 or bf16")
+    if not (base_input.is_cuda):
+        raise RuntimeError("base_input must be CUDA")
+    if not (base_input.is_contiguous()):
+        raise RuntimeError("base_input must be contiguous")
+    if base_input.dim() != 3:
+        raise RuntimeError("base_input must be 3-D [B, d_model, L]")
+    if base_input.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+        raise RuntimeError("base_input must be fp32, fp16 or bf16")
     B, Dm, L = base_input.shape
     dev = base_input.device
-    with torch.cuda.device(dev):
+    with _nat.on_device(dev):
         x2d = base_input.view(B * Dm, L)
         bitmask, counts, cu, meta = _count_scan(x2d, _nat.dtype_code(base_input.dtype), threshold)
         E, max_seqlen = meta.wait(dev)
@@ -109,23 +107,27 @@ def expand_base_events(base_ch_ids, base_t_steps, base_k_flat, base_cu_seqlens, 
     """Replicate base channel c into logical channels c*expand + r
     (repeat_interleave order) -> [channel_ids, time_steps, k_flat,
     cu_seqlens, max_seqlen] (extract_events_cuda.cu:529-603)."""
-    _check(base_ch_ids.is_cuda, "base_ch_ids must be CUDA")
-    _check(base_ch_ids.is_contiguous(), "base_ch_ids must be contiguous")
+    if not (base_ch_ids.is_cuda):
+        raise RuntimeError("base_ch_ids must be CUDA")
+    if not (base_ch_ids.is_contiguous()):
+        raise RuntimeError("base_ch_ids must be contiguous")
     NC_base = int(B) * int(d_model)
     NC_inner = NC_base * int(expand)
     E_base = int(base_ch_ids.size(0))
     dev = base_ch_ids.device
-    with torch.cuda.device(dev):
+    with _nat.on_device(dev):
         if E_base == 0:
             ei = torch.zeros(0, dtype=_I32, device=dev)
             return [ei, ei, ei, torch.zeros(NC_inner + 1, dtype=_I32, device=dev),
                     torch.zeros(1, dtype=_I32, device=dev)]
         for name, tns in (("base_t_steps", base_t_steps), ("base_k_flat", base_k_flat),
                           ("base_cu_seqlens", base_cu_seqlens)):
-            _check(tns.is_cuda and tns.dtype == _I32 and tns.is_contiguous(),
-                   f"{name} must be a contiguous int32 CUDA tensor")
-        _check(base_ch_ids.dtype == _I32, "base_ch_ids must be int32")
-        _check(base_cu_seqlens.numel() >= NC_base + 1, "base_cu_seqlens must have B*d_model+1 entries")
+            if not (tns.is_cuda and tns.dtype == _I32 and tns.is_contiguous()):
+                raise RuntimeError(f"{name} must be a contiguous int32 CUDA tensor")
+        if base_ch_ids.dtype != _I32:
+            raise RuntimeError("base_ch_ids must be int32")
+        if base_cu_seqlens.numel() < NC_base + 1:
+            raise RuntimeError("base_cu_seqlens must have B*d_model+1 entries")
         E = E_base * int(expand)
         ch, t, k = _empty_i32(E, dev), _empty_i32(E, dev), _empty_i32(E, dev)
         cu = _empty_i32(NC_inner + 1, dev)
@@ -144,12 +146,15 @@ def expand_base_events(base_ch_ids, base_t_steps, base_k_flat, base_cu_seqlens, 
 def extract_events(mask):
     """LEGACY: bool mask [B, D, L] -> [ch_ids, t_steps, k_flat, cu_seqlens,
     max_seqlen, head_flags] (extract_events_cuda.cu:117-179)."""
-    _check(mask.is_cuda, "mask must be a CUDA tensor")
-    _check(mask.is_contiguous(), "mask must be contiguous")
-    _check(mask.dtype == torch.bool, "mask must be bool")
+    if not (mask.is_cuda):
+        raise RuntimeError("mask must be a CUDA tensor")
+    if not (mask.is_contiguous()):
+        raise RuntimeError("mask must be contiguous")
+    if mask.dtype != torch.bool:
+        raise RuntimeError("mask must be bool")
     B, D, L = mask.shape
     dev = mask.device
-    with torch.cuda.device(dev):
+    with _nat.on_device(dev):
         x2d = mask.view(B * D, L)
         bitmask, counts, cu, meta = _count_scan(x2d, _nat.U8, 0.5)
         E, max_seqlen = meta.wait(dev)
@@ -166,17 +171,22 @@ def extract_events(mask):
 def gather_events_fwd(x, channel_ids, time_steps):
     """out_x[e] = x.view(NC, L)[channel_ids[e], time_steps[e]] -> [out_x]
     (extract_events_cuda.cu:670-708)."""
-    _check(x.is_cuda, "gather_events_fwd: x must be a CUDA tensor")
-    _check(x.is_contiguous(), "gather_events_fwd: x must be contiguous")
-    _check(channel_ids.dtype == _I32, "gather_events_fwd: channel_ids must be int32")
-    _check(time_steps.dtype == _I32, "gather_events_fwd: time_steps must be int32")
-    _check(x.dim() == 3, "gather_events_fwd: x must be 3-D [B, D, L]")
+    if not (x.is_cuda):
+        raise RuntimeError("gather_events_fwd: x must be a CUDA tensor")
+    if not (x.is_contiguous()):
+        raise RuntimeError("gather_events_fwd: x must be contiguous")
+    if channel_ids.dtype != _I32:
+        raise RuntimeError("gather_events_fwd: channel_ids must be int32")
+    if time_steps.dtype != _I32:
+        raise RuntimeError("gather_events_fwd: time_steps must be int32")
+    if x.dim() != 3:
+        raise RuntimeError("gather_events_fwd: x must be 3-D [B, D, L]")
     B, D, L = x.shape
     E = int(channel_ids.size(0))
     out = torch.empty(E, dtype=x.dtype, device=x.device)
     if E == 0:
         return [out]
-    with torch.cuda.device(x.device):
+    with _nat.on_device(x.device):
         _nat.call("bcm_gather_fwd", _nat.ptr(x), _nat.dtype_code(x.dtype), B * D, L,
                   _nat.ptr(channel_ids.contiguous()), _nat.ptr(time_steps.contiguous()), E,
                   _nat.ptr(out), _nat.stream_of(x))
@@ -189,12 +199,15 @@ def gather_events_bwd(grad_x, channel_ids, time_steps, NC, L):
     For the streams of extract_base_events (unchanged), dx is written row
     by row from the extraction's event index (bcm_gather_bwd_rows: no zero
     pass, no scatter; the same values)."""
-    _check(grad_x.is_cuda, "gather_events_bwd: grad tensor must be CUDA")
-    _check(channel_ids.dtype == _I32, "gather_events_bwd: channel_ids must be int32")
-    _check(time_steps.dtype == _I32, "gather_events_bwd: time_steps must be int32")
+    if not (grad_x.is_cuda):
+        raise RuntimeError("gather_events_bwd: grad tensor must be CUDA")
+    if channel_ids.dtype != _I32:
+        raise RuntimeError("gather_events_bwd: channel_ids must be int32")
+    if time_steps.dtype != _I32:
+        raise RuntimeError("gather_events_bwd: time_steps must be int32")
     NC, L = int(NC), int(L)
     dx = torch.empty((NC, L), dtype=grad_x.dtype, device=grad_x.device)
-    with torch.cuda.device(grad_x.device):
+    with _nat.on_device(grad_x.device):
         g = grad_x.contiguous()
         idx = _prov.event_index_for(time_steps, None, L, channel_ids)
         if (idx is not None and idx[0].size(0) == NC and g.dim() == 1 and g.size(0) == time_steps.size(0)
@@ -212,7 +225,7 @@ def _extract_indexed_exact(base_input, threshold, expand, x, positions):
     before the fill, which then writes exactly E events."""
     B, Dm, L = base_input.shape
     dev = base_input.device
-    with torch.cuda.device(dev):
+    with _nat.on_device(dev):
         x2d = base_input.view(B * Dm, L)
         bitmask, counts, base_cu, meta = _count_scan(x2d, _nat.dtype_code(base_input.dtype), threshold)
         E_base, max_seqlen = meta.wait(dev)
@@ -240,12 +253,14 @@ def spike_bits(p, threshold, want_s=True):
     returns (s, bitmask) with s = (p >= threshold) + p - p (None unless
     want_s) and the event bitmask [B*Dm, words] of the transposed spikes,
     ready for extract_events_indexed(bits=...)."""
-    _check(p.is_cuda and p.is_contiguous() and p.dim() == 3, "p must be a contiguous 3-D CUDA tensor [B, L, Dm]")
-    _check(p.dtype in (torch.float32, torch.float16, torch.bfloat16), "p must be fp32, fp16 or bf16")
+    if not (p.is_cuda and p.is_contiguous() and p.dim() == 3):
+        raise RuntimeError("p must be a contiguous 3-D CUDA tensor [B, L, Dm]")
+    if p.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+        raise RuntimeError("p must be fp32, fp16 or bf16")
     B, L, Dm = p.shape
     bitmask = torch.empty((B * Dm, _nat.bitmask_words(L)), dtype=_I32, device=p.device)
     s = torch.empty_like(p) if want_s else None
-    with torch.cuda.device(p.device):
+    with _nat.on_device(p.device):
         _nat.call("bcm_spike_bits", _nat.ptr(p), _nat.dtype_code(p.dtype), B, L, Dm, float(threshold),
                   _nat.ptr(bitmask), _nat.ptr(s), _nat.stream_of(p))
     return s, bitmask
@@ -283,30 +298,34 @@ def extract_events_indexed(base_input, threshold, expand=1, x=None, positions=Tr
     then not read and may be None, and the count pass only counts bits."""
     if bits is not None:
         bits_mask, (B, Dm, L) = bits
-        _check(bits_mask.is_cuda and bits_mask.dtype == _I32 and bits_mask.is_contiguous()
-               and tuple(bits_mask.shape) == (B * Dm, _nat.bitmask_words(L)), "bits must be [B*d_model, words] int32")
-        _check(not exact_alloc and B * Dm > 0 and L > 0, "bits need the fused fill and a non-empty batch")
+        if not (bits_mask.is_cuda and bits_mask.dtype == _I32 and bits_mask.is_contiguous()
+                and tuple(bits_mask.shape) == (B * Dm, _nat.bitmask_words(L))):
+            raise RuntimeError("bits must be [B*d_model, words] int32")
+        if not (not exact_alloc and B * Dm > 0 and L > 0):
+            raise RuntimeError("bits need the fused fill and a non-empty batch")
         dev = bits_mask.device
     else:
-        _check(base_input.is_cuda and base_input.is_contiguous() and base_input.dim() == 3,
-               "base_input must be a contiguous 3-D CUDA tensor [B, d_model, L]")
+        if not (base_input.is_cuda and base_input.is_contiguous() and base_input.dim() == 3):
+            raise RuntimeError("base_input must be a contiguous 3-D CUDA tensor [B, d_model, L]")
         B, Dm, L = base_input.shape
         dev = base_input.device
     expand = int(expand)
     NC = B * Dm
     if conv is not None:
-        _check(x is not None and x.is_cuda and x.dim() == 3 and tuple(x.shape) == (B, Dm * expand, L)
-               and x.stride(2) == 1, "x must be a CUDA tensor [B, d_model*expand, L] with contiguous rows")
-        _check(not exact_alloc, "conv needs the fused fill (exact_alloc=False)")
+        if not (x is not None and x.is_cuda and x.dim() == 3 and tuple(x.shape) == (B, Dm * expand, L)
+                and x.stride(2) == 1):
+            raise RuntimeError("x must be a CUDA tensor [B, d_model*expand, L] with contiguous rows")
+        if exact_alloc:
+            raise RuntimeError("conv needs the fused fill (exact_alloc=False)")
         if NC == 0 or L == 0:
             r = _extract_indexed_exact(base_input, threshold, expand, None, positions)
             return r[:5] + (torch.empty(0, dtype=x.dtype, device=dev),) + r[6:]
     elif x is not None:
-        _check(x.is_cuda and x.is_contiguous() and tuple(x.shape) == (B, Dm * expand, L),
-               "x must be a contiguous CUDA tensor [B, d_model*expand, L]")
+        if not (x.is_cuda and x.is_contiguous() and tuple(x.shape) == (B, Dm * expand, L)):
+            raise RuntimeError("x must be a contiguous CUDA tensor [B, d_model*expand, L]")
     if exact_alloc or NC == 0 or L == 0:
         return _extract_indexed_exact(base_input, threshold, expand, x, positions)
-    with torch.cuda.device(dev):
+    with _nat.on_device(dev):
         s = _nat.stream_of(bits[0] if bits is not None else base_input)
         NCi, cap = NC * expand, NC * expand * L
         bitmask = bits[0] if bits is not None else torch.empty((NC, _nat.bitmask_words(L)), dtype=_I32, device=dev)
@@ -332,7 +351,8 @@ def extract_events_indexed(base_input, threshold, expand=1, x=None, positions=Tr
             w, b, silu = conv
             w = w.detach().float().contiguous()
             b = b.detach().float().contiguous() if b is not None else None
-            _check(w.dim() == 2 and w.size(0) == Dm * expand and 1 <= w.size(1) <= 8, "conv weight must be [D, K<=8]")
+            if not (w.dim() == 2 and w.size(0) == Dm * expand and 1 <= w.size(1) <= 8):
+                raise RuntimeError("conv weight must be [D, K<=8]")
             _nat.call("bcm_extract_fill_blocks_conv", _nat.ptr(bitmask), _nat.ptr(counts), _nat.ptr(bsums),
                       meta.ptr(), NC, L, expand, _nat.ptr(x), _nat.dtype_code(x.dtype), x.stride(0), x.stride(1),
                       Dm * expand, _nat.ptr(w), _nat.ptr(b), int(w.size(1)), int(bool(silu)), _nat.ptr(cu),

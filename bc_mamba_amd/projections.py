@@ -30,6 +30,7 @@ SPLIT = 8
 MIN_TOKENS = 8192
 
 
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 _LIMIT = 2 ** 31  # bytes: the kernel's 32-bit offsets
 
 
@@ -48,18 +49,19 @@ def _kernel_form(x, y, bias=None):
     product stays with torch: other types and devices, a product that
     autograd must see (no custom backward around it), autocast, a traced or
     wrapped tensor, strides without a contiguous dimension, an operand of 2 GiB."""
-    ts = (x, y) if bias is None else (x, y, bias)
-    for t in ts:
-        if type(t) not in (torch.Tensor, torch.nn.Parameter) or t.dtype != torch.float32 or not t.is_cuda:
+    grad = torch.is_grad_enabled()
+    for t in (x, y) if bias is None else (x, y, bias):
+        if (type(t) not in _PLAIN or t.dtype != torch.float32 or not t.is_cuda or t.device != x.device
+                or (grad and t.requires_grad)):
             return None
-    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
-        return None
     if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling():
         return None
-    if any(t.device != x.device for t in ts) or x.dim() != 2 or y.dim() != 2 or x.size(1) != y.size(0):
+    if x.dim() != 2 or y.dim() != 2 or x.size(1) != y.size(0):
         return None
     (M, K), N = x.shape, y.size(1)
-    if M == 0 or N == 0 or K == 0 or (bias is not None and (bias.dim() != 1 or bias.size(0) != N or bias.stride(0) != 1)):
+    if M == 0 or N == 0 or K == 0:
+        return None
+    if bias is not None and (bias.dim() != 1 or bias.size(0) != N or bias.stride(0) != 1):
         return None
     fx, fy = _major(x, M, K), _major(y, K, N)
     if fx is None or fy is None:
@@ -78,10 +80,14 @@ def mm(x, y, bias=None):
     form = _kernel_form(x, y, bias)
     if form is None:
         return x @ y if bias is None else torch.addmm(bias, x, y)
+    return _kernel_mm(x, y, bias, form)
+
+
+def _kernel_mm(x, y, bias, form):
     x_k, ldx, y_k, ldy = form
     (M, K), N = x.shape, y.size(1)
     out = torch.empty((M, N), dtype=torch.float32, device=x.device)
-    with torch.cuda.device(x.device):
+    with _nat.on_device(x.device):
         nbytes = 0 if bias is not None else int(_nat.lib().bcm_gemm_f32_workspace_bytes(M, N, K))
         ws = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device) if nbytes else None
         _nat.call("bcm_gemm_f32", x.data_ptr(), int(x_k), ldx, y.data_ptr(), int(y_k), ldy,
@@ -98,8 +104,9 @@ def weight_grad(g, x, tokens_first=True):
     """Σ over tokens of g ⊗ x: gᵀ @ x for g [M, N] (tokens_first) or g @ x
     for g [N, M], with x [M, K]."""
     gt = g.t() if tokens_first else g
-    if _kernel_form(gt, x) is not None:
-        return mm(gt, x)
+    form = _kernel_form(gt, x)
+    if form is not None:
+        return _kernel_mm(gt, x, None, form)
     m = x.size(0)
     if not _split_ok(m, g, x):
         return gt @ x
@@ -117,9 +124,10 @@ class _LinearFn(torch.autograd.Function):
         ctx.save_for_backward(x, weight)
         ctx.has_bias = bias is not None
         if x.dim() > 1 and x.is_contiguous():
-            x2 = x.view(-1, x.size(-1)) if x.numel() else x
-            if _kernel_form(x2, weight.t(), bias) is not None:
-                return mm(x2, weight.t(), bias).view(*x.shape[:-1], weight.size(0))
+            x2, wt = x.view(-1, x.size(-1)) if x.numel() else x, weight.t()
+            form = _kernel_form(x2, wt, bias)
+            if form is not None:
+                return _kernel_mm(x2, wt, bias, form).view(*x.shape[:-1], weight.size(0))
         return F.linear(x, weight, bias)
 
     @staticmethod

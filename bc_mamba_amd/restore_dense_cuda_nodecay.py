@@ -27,11 +27,6 @@ __all__ = ["restore_dense_fwd", "restore_dense_bwd", "build_event_index", "resto
 _FLOATS = (torch.float32, torch.float16, torch.bfloat16)
 
 
-def _check(cond, msg):
-    if not cond:
-        raise RuntimeError(msg)
-
-
 def build_event_index(time_steps, cu_seqlens, seqlen, zero_f32=None):
     """(bitmask, tile_start) of per-channel sorted time steps; optionally
     zero-fills the float32 tensor zero_f32 in the same launch."""
@@ -115,9 +110,12 @@ def restore_proj_fwd_indexed(y_flat, event_index, n_ch, dim, seqlen, weight, bia
     restore output (bcm_restore_proj_fwd): F.linear(restore(y_flat), weight,
     bias) as (B, L, d_model) float32. fp32 y_flat, weight and bias."""
     fn = "restore_proj_fwd_indexed"
-    _check(y_flat.dtype == torch.float32 and weight.dtype == torch.float32, f"{fn}: fp32 y_flat and weight")
-    _check(bias is None or bias.dtype == torch.float32, f"{fn}: fp32 bias")
-    _check(weight.dim() == 2 and weight.size(1) == dim and weight.is_contiguous(), f"{fn}: weight [d_model, dim]")
+    if not (y_flat.dtype == torch.float32 and weight.dtype == torch.float32):
+        raise RuntimeError(f"{fn}: fp32 y_flat and weight")
+    if not (bias is None or bias.dtype == torch.float32):
+        raise RuntimeError(f"{fn}: fp32 bias")
+    if not (weight.dim() == 2 and weight.size(1) == dim and weight.is_contiguous()):
+        raise RuntimeError(f"{fn}: weight [d_model, dim]")
     bitmask, tile_start, mrd = event_index
     dm = weight.size(0)
     out = torch.empty((n_ch // dim, seqlen, dm), dtype=torch.float32, device=y_flat.device)
@@ -150,30 +148,44 @@ def restore_proj_bwd_indexed(dout, y_flat, event_index, n_ch, dim, seqlen, weigh
 def restore_dense_fwd(y_flat, time_steps, cu_seqlens, dim, seqlen, out_dtype=None):
     """Zero-order-hold restore forward (restore_dense.cpp:43-130)."""
     fn = "restore_dense_fwd"
-    _check(y_flat.dtype in _FLOATS, f"{fn}: y_flat must be fp32, fp16, or bf16")
-    _check(time_steps.dtype == torch.int32, f"{fn}: time_steps must be int32 (torch.int32)")
-    _check(cu_seqlens.dtype == torch.int32, f"{fn}: cu_seqlens must be int32 (torch.int32)")
-    _check(y_flat.is_cuda and time_steps.is_cuda and cu_seqlens.is_cuda, f"{fn}: all tensors must be on CUDA")
-    _check(y_flat.is_contiguous() and time_steps.is_contiguous() and cu_seqlens.is_contiguous(),
-           f"{fn}: all tensors must be contiguous")
-    _check(y_flat.dim() == 1, f"{fn}: y_flat must be 1-D")
-    _check(time_steps.shape == y_flat.shape, f"{fn}: time_steps shape must equal y_flat shape")
-    _check(cu_seqlens.dim() == 1, f"{fn}: cu_seqlens must be 1-D")
+    if y_flat.dtype not in _FLOATS:
+        raise RuntimeError(f"{fn}: y_flat must be fp32, fp16, or bf16")
+    if time_steps.dtype != torch.int32:
+        raise RuntimeError(f"{fn}: time_steps must be int32 (torch.int32)")
+    if cu_seqlens.dtype != torch.int32:
+        raise RuntimeError(f"{fn}: cu_seqlens must be int32 (torch.int32)")
+    if not (y_flat.is_cuda and time_steps.is_cuda and cu_seqlens.is_cuda):
+        raise RuntimeError(f"{fn}: all tensors must be on CUDA")
+    if not (y_flat.is_contiguous() and time_steps.is_contiguous() and cu_seqlens.is_contiguous()):
+        raise RuntimeError(f"{fn}: all tensors must be contiguous")
+    if y_flat.dim() != 1:
+        raise RuntimeError(f"{fn}: y_flat must be 1-D")
+    if time_steps.shape != y_flat.shape:
+        raise RuntimeError(f"{fn}: time_steps shape must equal y_flat shape")
+    if cu_seqlens.dim() != 1:
+        raise RuntimeError(f"{fn}: cu_seqlens must be 1-D")
     dim, seqlen = int(dim), int(seqlen)
-    _check(dim >= 1, f"{fn}: dim must be >= 1")
-    _check(seqlen >= 1, f"{fn}: seqlen must be >= 1")
+    if dim < 1:
+        raise RuntimeError(f"{fn}: dim must be >= 1")
+    if seqlen < 1:
+        raise RuntimeError(f"{fn}: seqlen must be >= 1")
     n_ch = int(cu_seqlens.size(0)) - 1
-    _check(n_ch >= 1, f"{fn}: cu_seqlens must have at least 2 elements")
-    _check(n_ch % dim == 0, f"{fn}: n_channels (B*D) must be divisible by dim")
+    if n_ch < 1:
+        raise RuntimeError(f"{fn}: cu_seqlens must have at least 2 elements")
+    if n_ch % dim != 0:
+        raise RuntimeError(f"{fn}: n_channels (B*D) must be divisible by dim")
     out_dtype = y_flat.dtype if out_dtype is None else out_dtype
-    _check(out_dtype in _FLOATS, f"{fn}: out_dtype must be fp32, fp16, or bf16")
+    if out_dtype not in _FLOATS:
+        raise RuntimeError(f"{fn}: out_dtype must be fp32, fp16, or bf16")
     if y_flat.dtype == torch.float16:
-        _check(out_dtype == torch.float16, f"{fn}: fp16 input only supports fp16 output")
+        if out_dtype != torch.float16:
+            raise RuntimeError(f"{fn}: fp16 input only supports fp16 output")
     if y_flat.dtype == torch.bfloat16:
-        _check(out_dtype == torch.bfloat16, f"{fn}: bf16 input only supports bf16 output")
+        if out_dtype != torch.bfloat16:
+            raise RuntimeError(f"{fn}: bf16 input only supports bf16 output")
     if y_flat.numel() == 0:  # no events: every position precedes its channel's first event
         return torch.zeros((n_ch // dim, seqlen, dim), dtype=out_dtype, device=y_flat.device)
-    with torch.cuda.device(y_flat.device):
+    with _nat.on_device(y_flat.device):
         idx = _prov.event_index_for(time_steps, cu_seqlens, seqlen)  # the extraction's own, when unchanged
         bitmask, tile_start = idx if idx is not None else build_event_index(time_steps, cu_seqlens, seqlen)
         return restore_fwd_indexed(y_flat, (bitmask, tile_start, 1), n_ch, dim, seqlen, out_dtype)
@@ -183,24 +195,34 @@ def restore_dense_bwd(dout, time_steps, cu_seqlens, dim, seqlen):
     """Zero-order-hold restore backward -> dy (E,) float32
     (restore_dense.cpp:138-202)."""
     fn = "restore_dense_bwd"
-    _check(dout.dtype in _FLOATS, f"{fn}: dout must be fp32/fp16/bf16")
-    _check(time_steps.dtype == torch.int32, f"{fn}: time_steps must be int32")
-    _check(cu_seqlens.dtype == torch.int32, f"{fn}: cu_seqlens must be int32")
-    _check(dout.is_cuda and time_steps.is_cuda and cu_seqlens.is_cuda, f"{fn}: all tensors must be on CUDA")
-    _check(dout.is_contiguous() and time_steps.is_contiguous() and cu_seqlens.is_contiguous(),
-           f"{fn}: all tensors must be contiguous")
+    if dout.dtype not in _FLOATS:
+        raise RuntimeError(f"{fn}: dout must be fp32/fp16/bf16")
+    if time_steps.dtype != torch.int32:
+        raise RuntimeError(f"{fn}: time_steps must be int32")
+    if cu_seqlens.dtype != torch.int32:
+        raise RuntimeError(f"{fn}: cu_seqlens must be int32")
+    if not (dout.is_cuda and time_steps.is_cuda and cu_seqlens.is_cuda):
+        raise RuntimeError(f"{fn}: all tensors must be on CUDA")
+    if not (dout.is_contiguous() and time_steps.is_contiguous() and cu_seqlens.is_contiguous()):
+        raise RuntimeError(f"{fn}: all tensors must be contiguous")
     dim, seqlen = int(dim), int(seqlen)
-    _check(dim >= 1, f"{fn}: dim must be >= 1")
-    _check(seqlen >= 1, f"{fn}: seqlen must be >= 1")
+    if dim < 1:
+        raise RuntimeError(f"{fn}: dim must be >= 1")
+    if seqlen < 1:
+        raise RuntimeError(f"{fn}: seqlen must be >= 1")
     n_ch = int(cu_seqlens.size(0)) - 1
-    _check(dout.dim() == 3, f"{fn}: dout must be 3-D (B, L, D)")
-    _check(dout.size(1) == seqlen, f"{fn}: dout.size(1) must equal seqlen")
-    _check(dout.size(2) == dim, f"{fn}: dout.size(2) must equal dim (D)")
-    _check(dout.size(0) * dim == n_ch, f"{fn}: dout.size(0)*dim must equal n_channels")
+    if dout.dim() != 3:
+        raise RuntimeError(f"{fn}: dout must be 3-D (B, L, D)")
+    if dout.size(1) != seqlen:
+        raise RuntimeError(f"{fn}: dout.size(1) must equal seqlen")
+    if dout.size(2) != dim:
+        raise RuntimeError(f"{fn}: dout.size(2) must equal dim (D)")
+    if dout.size(0) * dim != n_ch:
+        raise RuntimeError(f"{fn}: dout.size(0)*dim must equal n_channels")
     dy = torch.empty(int(time_steps.size(0)), dtype=torch.float32, device=dout.device)
     if dy.numel() == 0:
         return dy
-    with torch.cuda.device(dout.device):
+    with _nat.on_device(dout.device):
         idx = _prov.event_index_for(time_steps, cu_seqlens, seqlen)
         if idx is not None:  # the extraction's index: every event is in it, no zero-fill
             restore_bwd_indexed(dout, idx + (1,), n_ch, dim, seqlen, dy)

@@ -31,11 +31,6 @@ __all__ = ["fwd_flat_ch", "bwd_flat_ch"]
 _FLOATS = (torch.float32, torch.float16, torch.bfloat16)
 
 
-def _check(cond, msg):
-    if not cond:
-        raise RuntimeError(msg)
-
-
 def n_chunks_for(max_seqlen):
     """Chunk count of the saved state x: max(1, ceil(max_seqlen / 2048))."""
     return max(1, (int(max_seqlen) + 2047) // 2048)
@@ -45,72 +40,111 @@ def _common_checks(fn, u_flat, k_flat, cu_seqlens, max_seqlen, dt_idle, dt_activ
                    tile_offsets, is_depthwise_bc, pw_B, pw_C, extra_cuda=(), bwd=False, tile_chunk_size=0):
     """The reference's checks (selective_scan.cpp:697-781, 939-998); returns
     (dim, dstate, mode) with mode "depthwise", "tiled" or "legacy"."""
-    _check(u_flat.dtype in _FLOATS, f"{fn}: u_flat must be fp16/bf16/fp32")
-    _check(A.dtype == torch.float32, f"{fn}: A must be float32")
-    _check(B.dtype == torch.float32, f"{fn}: B must be float32")
-    _check(C.dtype == torch.float32, f"{fn}: C must be float32")
-    _check(all(t.is_cuda for t in (u_flat, k_flat, cu_seqlens, dt_idle, dt_active, A, B, C, *extra_cuda)),
-           f"{fn}: all tensors must be CUDA tensors")
-    _check(u_flat.dim() == 1, f"{fn}: u_flat must be 1-D")
-    _check(k_flat.dim() == 1, f"{fn}: k_flat must be 1-D")
-    _check(cu_seqlens.dim() == 1, f"{fn}: cu_seqlens must be 1-D")
-    _check(k_flat.dtype == torch.int32, f"{fn}: k_flat must be int32")
-    _check(cu_seqlens.dtype == torch.int32, f"{fn}: cu_seqlens must be int32")
-    _check(k_flat.size(0) == u_flat.size(0), f"{fn}: k_flat must match u_flat shape")
-    _check(cu_seqlens.size(0) >= 2, f"{fn}: cu_seqlens must have at least 2 elements")
-    _check(dt_idle.dtype == torch.float32 and dt_active.dtype == torch.float32,
-           f"{fn}: dt_idle/dt_active must be float32")
-    _check(dt_idle.dim() == 1 and dt_active.dim() == 1, f"{fn}: dt_idle/dt_active must be 1-D")
-    _check(A.dim() == 2, f"{fn}: A must be 2-D (dim, dstate)")
+    if u_flat.dtype not in _FLOATS:
+        raise RuntimeError(f"{fn}: u_flat must be fp16/bf16/fp32")
+    if A.dtype != torch.float32:
+        raise RuntimeError(f"{fn}: A must be float32")
+    if B.dtype != torch.float32:
+        raise RuntimeError(f"{fn}: B must be float32")
+    if C.dtype != torch.float32:
+        raise RuntimeError(f"{fn}: C must be float32")
+    if not all(t.is_cuda for t in (u_flat, k_flat, cu_seqlens, dt_idle, dt_active, A, B, C, *extra_cuda)):
+        raise RuntimeError(f"{fn}: all tensors must be CUDA tensors")
+    if u_flat.dim() != 1:
+        raise RuntimeError(f"{fn}: u_flat must be 1-D")
+    if k_flat.dim() != 1:
+        raise RuntimeError(f"{fn}: k_flat must be 1-D")
+    if cu_seqlens.dim() != 1:
+        raise RuntimeError(f"{fn}: cu_seqlens must be 1-D")
+    if k_flat.dtype != torch.int32:
+        raise RuntimeError(f"{fn}: k_flat must be int32")
+    if cu_seqlens.dtype != torch.int32:
+        raise RuntimeError(f"{fn}: cu_seqlens must be int32")
+    if k_flat.size(0) != u_flat.size(0):
+        raise RuntimeError(f"{fn}: k_flat must match u_flat shape")
+    if cu_seqlens.size(0) < 2:
+        raise RuntimeError(f"{fn}: cu_seqlens must have at least 2 elements")
+    if not (dt_idle.dtype == torch.float32 and dt_active.dtype == torch.float32):
+        raise RuntimeError(f"{fn}: dt_idle/dt_active must be float32")
+    if not (dt_idle.dim() == 1 and dt_active.dim() == 1):
+        raise RuntimeError(f"{fn}: dt_idle/dt_active must be 1-D")
+    if A.dim() != 2:
+        raise RuntimeError(f"{fn}: A must be 2-D (dim, dstate)")
     dim, dstate = A.shape
-    _check(dstate <= 256, f"{fn}: dstate must be <= 256")
-    _check(tuple(dt_idle.shape) == (dim,), f"{fn}: dt_idle must have shape ({dim},)")
-    _check(tuple(dt_active.shape) == (dim,), f"{fn}: dt_active must have shape ({dim},)")
+    if dstate > 256:
+        raise RuntimeError(f"{fn}: dstate must be <= 256")
+    if tuple(dt_idle.shape) != (dim,):
+        raise RuntimeError(f"{fn}: dt_idle must have shape ({dim},)")
+    if tuple(dt_active.shape) != (dim,):
+        raise RuntimeError(f"{fn}: dt_active must have shape ({dim},)")
     E = int(u_flat.size(0))
     use_tiled = tile_offsets is not None
     if is_depthwise_bc and not use_tiled:
-        _check(B.dim() == 2 and C.dim() == 2, f"{fn} (depthwise): W_B/W_C must be 2-D [dim, dstate]")
-        _check(tuple(B.shape) == (dim, dstate), f"{fn} (depthwise): W_B must be [dim, dstate]")
-        _check(tuple(C.shape) == (dim, dstate), f"{fn} (depthwise): W_C must be [dim, dstate]")
-        _check(B.is_contiguous() and C.is_contiguous(), f"{fn} (depthwise): W_B/W_C must be contiguous")
+        if not (B.dim() == 2 and C.dim() == 2):
+            raise RuntimeError(f"{fn} (depthwise): W_B/W_C must be 2-D [dim, dstate]")
+        if tuple(B.shape) != (dim, dstate):
+            raise RuntimeError(f"{fn} (depthwise): W_B must be [dim, dstate]")
+        if tuple(C.shape) != (dim, dstate):
+            raise RuntimeError(f"{fn} (depthwise): W_C must be [dim, dstate]")
+        if not (B.is_contiguous() and C.is_contiguous()):
+            raise RuntimeError(f"{fn} (depthwise): W_B/W_C must be contiguous")
         if pw_B is not None:
-            _check(pw_C is not None, f"{fn}: pw_C is required with pw_B")
-            _check(pw_B.dtype == torch.float32 and pw_C.dtype == torch.float32, f"{fn}: pw_B/pw_C must be float32")
-            _check(pw_B.is_cuda and pw_C.is_cuda and pw_B.is_contiguous() and pw_C.is_contiguous(),
-                   f"{fn}: pw_B/pw_C must be CUDA and contiguous")
-            _check(pw_B.dim() == 2 and tuple(pw_B.shape) == (dim, dim), f"{fn}: pw_B must be [dim, dim]")
-            _check(pw_C.dim() == 2 and tuple(pw_C.shape) == (dim, dim), f"{fn}: pw_C must be [dim, dim]")
+            if pw_C is None:
+                raise RuntimeError(f"{fn}: pw_C is required with pw_B")
+            if not (pw_B.dtype == torch.float32 and pw_C.dtype == torch.float32):
+                raise RuntimeError(f"{fn}: pw_B/pw_C must be float32")
+            if not (pw_B.is_cuda and pw_C.is_cuda and pw_B.is_contiguous() and pw_C.is_contiguous()):
+                raise RuntimeError(f"{fn}: pw_B/pw_C must be CUDA and contiguous")
+            if not (pw_B.dim() == 2 and tuple(pw_B.shape) == (dim, dim)):
+                raise RuntimeError(f"{fn}: pw_B must be [dim, dim]")
+            if not (pw_C.dim() == 2 and tuple(pw_C.shape) == (dim, dim)):
+                raise RuntimeError(f"{fn}: pw_C must be [dim, dim]")
         mode = "depthwise"
     elif use_tiled:
-        _check(B.dim() == 3 and C.dim() == 3, f"{fn}: tiled B/C must be 3-D [N_tiles, dstate, tile_chunk_size]")
-        _check(B.size(1) == dstate and C.size(1) == dstate, f"{fn}: tiled B/C dim-1 must equal dstate")
-        _check(B.is_contiguous() and C.is_contiguous(), f"{fn}: tiled B/C must be contiguous")
-        _check(int(tile_chunk_size) >= 1 and B.size(2) == int(tile_chunk_size) and C.size(2) == int(tile_chunk_size),
-               f"{fn}: tiled B/C dim-2 must equal tile_chunk_size (>= 1)")
-        _check(B.size(0) == C.size(0), f"{fn}: tiled B and C must have the same number of tiles")
-        _check(tile_offsets.is_cuda and tile_offsets.dtype == torch.int32 and tile_offsets.dim() == 1
-               and tile_offsets.is_contiguous() and tile_offsets.size(0) >= cu_seqlens.size(0) - 1,
-               f"{fn}: tile_offsets must be a contiguous int32 CUDA tensor with one entry per channel")
+        if not (B.dim() == 3 and C.dim() == 3):
+            raise RuntimeError(f"{fn}: tiled B/C must be 3-D [N_tiles, dstate, tile_chunk_size]")
+        if not (B.size(1) == dstate and C.size(1) == dstate):
+            raise RuntimeError(f"{fn}: tiled B/C dim-1 must equal dstate")
+        if not (B.is_contiguous() and C.is_contiguous()):
+            raise RuntimeError(f"{fn}: tiled B/C must be contiguous")
+        if not (int(tile_chunk_size) >= 1 and B.size(2) == int(tile_chunk_size)
+                and C.size(2) == int(tile_chunk_size)):
+            raise RuntimeError(f"{fn}: tiled B/C dim-2 must equal tile_chunk_size (>= 1)")
+        if B.size(0) != C.size(0):
+            raise RuntimeError(f"{fn}: tiled B and C must have the same number of tiles")
+        if not (tile_offsets.is_cuda and tile_offsets.dtype == torch.int32 and tile_offsets.dim() == 1
+                and tile_offsets.is_contiguous() and tile_offsets.size(0) >= cu_seqlens.size(0) - 1):
+            raise RuntimeError(
+                f"{fn}: tile_offsets must be a contiguous int32 CUDA tensor with one entry per channel")
         mode = "tiled"
     else:
         if not bwd:
-            _check(B.dim() == 2 and C.dim() == 2, f"{fn}: B/C must be 2-D (dstate, E) [transposed layout]")
-            _check(tuple(B.shape) == (dstate, E), f"{fn}: B must have shape ({dstate}, {E})")
-            _check(tuple(C.shape) == (dstate, E), f"{fn}: C must have shape ({dstate}, {E})")
-            _check(B.stride(1) == 1 and C.stride(1) == 1,
-                   f"{fn}: B/C must have contiguous last dimension (stride(1) == 1)")
+            if not (B.dim() == 2 and C.dim() == 2):
+                raise RuntimeError(f"{fn}: B/C must be 2-D (dstate, E) [transposed layout]")
+            if tuple(B.shape) != (dstate, E):
+                raise RuntimeError(f"{fn}: B must have shape ({dstate}, {E})")
+            if tuple(C.shape) != (dstate, E):
+                raise RuntimeError(f"{fn}: C must have shape ({dstate}, {E})")
+            if not (B.stride(1) == 1 and C.stride(1) == 1):
+                raise RuntimeError(f"{fn}: B/C must have contiguous last dimension (stride(1) == 1)")
         else:
-            _check(B.dim() == 2 and C.dim() == 2, f"{fn}: B/C must be 2-D [dstate, E] or [dstate, dim]")
-            _check(B.stride(1) == 1 and C.stride(1) == 1, f"{fn}: B/C must have contiguous last dimension")
+            if not (B.dim() == 2 and C.dim() == 2):
+                raise RuntimeError(f"{fn}: B/C must be 2-D [dstate, E] or [dstate, dim]")
+            if not (B.stride(1) == 1 and C.stride(1) == 1):
+                raise RuntimeError(f"{fn}: B/C must have contiguous last dimension")
             for name, t in (("B", B), ("C", C)):
-                _check(t.size(0) == dstate and t.size(1) in (E, dim),
-                       f"{fn}: {name} must have shape ({dstate}, {E}) or ({dstate}, {dim})")
+                if not (t.size(0) == dstate and t.size(1) in (E, dim)):
+                    raise RuntimeError(f"{fn}: {name} must have shape ({dstate}, {E}) or ({dstate}, {dim})")
         mode = "legacy"
     if D is not None:
-        _check(D.dtype == torch.float32, f"{fn}: D must be float32")
-        _check(D.is_cuda and D.is_contiguous(), f"{fn}: D must be a contiguous CUDA tensor")
-        _check(tuple(D.shape) == (dim,), f"{fn}: D must have shape ({dim},)")
-    _check(int(max_seqlen) >= 0, f"{fn}: max_seqlen must be non-negative")
+        if D.dtype != torch.float32:
+            raise RuntimeError(f"{fn}: D must be float32")
+        if not (D.is_cuda and D.is_contiguous()):
+            raise RuntimeError(f"{fn}: D must be a contiguous CUDA tensor")
+        if tuple(D.shape) != (dim,):
+            raise RuntimeError(f"{fn}: D must have shape ({dim},)")
+    if int(max_seqlen) < 0:
+        raise RuntimeError(f"{fn}: max_seqlen must be non-negative")
     return dim, dstate, mode
 
 
@@ -148,8 +182,9 @@ def _acc_ptr(fn, acc, u_flat):
     """Device pointer of a per-event state-sum buffer (float32 [E]), or None."""
     if acc is None:
         return None
-    _check(acc.dtype == torch.float32 and acc.is_contiguous() and acc.numel() == u_flat.numel()
-           and acc.device == u_flat.device, f"{fn}: _acc must be a contiguous float32 (E,) tensor on u's device")
+    if not (acc.dtype == torch.float32 and acc.is_contiguous() and acc.numel() == u_flat.numel()
+            and acc.device == u_flat.device):
+        raise RuntimeError(f"{fn}: _acc must be a contiguous float32 (E,) tensor on u's device")
     return acc.data_ptr()
 
 
@@ -232,20 +267,23 @@ def fwd_flat_ch(u_flat, k_flat, cu_seqlens, max_seqlen, dt_idle, dt_active, A, B
     package's extraction (unchanged) with a max_seqlen at least its longest
     channel, which the extraction recorded on it."""
     fn = "selective_scan_fwd_flat_ch"
-    _check(u_flat.is_contiguous() and k_flat.is_contiguous() and cu_seqlens.is_contiguous(),
-           f"{fn}: u_flat/k_flat/cu_seqlens must be contiguous")
+    if not (u_flat.is_contiguous() and k_flat.is_contiguous() and cu_seqlens.is_contiguous()):
+        raise RuntimeError(f"{fn}: u_flat/k_flat/cu_seqlens must be contiguous")
     _, dstate, mode = _common_checks(fn, u_flat, k_flat, cu_seqlens, max_seqlen, dt_idle, dt_active, A, B, C, D,
                                      tile_offsets, is_depthwise_bc, pw_B, pw_C, tile_chunk_size=tile_chunk_size)
     if z is not None:
-        _check(z.dtype == u_flat.dtype, f"{fn}: z must have same dtype as u_flat")
-        _check(z.is_cuda and z.is_contiguous(), f"{fn}: z must be a contiguous CUDA tensor")
-        _check(z.dim() == 1 and z.size(0) == u_flat.size(0), f"{fn}: z must have shape (E,)")
+        if z.dtype != u_flat.dtype:
+            raise RuntimeError(f"{fn}: z must have same dtype as u_flat")
+        if not (z.is_cuda and z.is_contiguous()):
+            raise RuntimeError(f"{fn}: z must be a contiguous CUDA tensor")
+        if not (z.dim() == 1 and z.size(0) == u_flat.size(0)):
+            raise RuntimeError(f"{fn}: z must have shape (E,)")
     dev = u_flat.device
     n_ch = int(cu_seqlens.size(0)) - 1
     out = torch.empty_like(u_flat)
     x = torch.empty((n_ch, n_chunks_for(max_seqlen), dstate * 2), dtype=torch.float32, device=dev)
     out_z = torch.empty_like(u_flat) if z is not None else None
-    with torch.cuda.device(dev):
+    with _nat.on_device(dev):
         if mode == "depthwise" and pw_B is not None:
             B, C = pw_B @ B, pw_C @ C  # W_eff [dim, dstate]
         a = _args(u_flat, k_flat, cu_seqlens, max_seqlen, dt_idle.contiguous(), dt_active.contiguous(),
@@ -286,29 +324,37 @@ def bwd_flat_ch(u_flat, k_flat, cu_seqlens, max_seqlen, dt_idle, dt_active, A, B
     As fwd_flat_ch, raises RuntimeError when a channel holds more than
     max_seqlen events (unless `_trusted_seqlen`)."""
     fn = "selective_scan_bwd_flat_ch"
-    _check(dout_flat.dtype == u_flat.dtype, f"{fn}: dout_flat must match u_flat dtype")
-    _check(u_flat.is_contiguous() and k_flat.is_contiguous() and cu_seqlens.is_contiguous()
-           and dout_flat.is_contiguous(), f"{fn}: u_flat/k_flat/cu_seqlens/dout_flat must be contiguous")
-    _check(u_flat.dim() == 1 and k_flat.dim() == 1 and cu_seqlens.dim() == 1 and dout_flat.dim() == 1,
-           f"{fn}: u_flat/k_flat/cu_seqlens/dout_flat must be 1-D")
-    _check(dout_flat.size(0) == u_flat.size(0), f"{fn}: dout_flat must match u_flat shape")
+    if dout_flat.dtype != u_flat.dtype:
+        raise RuntimeError(f"{fn}: dout_flat must match u_flat dtype")
+    if not (u_flat.is_contiguous() and k_flat.is_contiguous() and cu_seqlens.is_contiguous()
+            and dout_flat.is_contiguous()):
+        raise RuntimeError(f"{fn}: u_flat/k_flat/cu_seqlens/dout_flat must be contiguous")
+    if not (u_flat.dim() == 1 and k_flat.dim() == 1 and cu_seqlens.dim() == 1 and dout_flat.dim() == 1):
+        raise RuntimeError(f"{fn}: u_flat/k_flat/cu_seqlens/dout_flat must be 1-D")
+    if dout_flat.size(0) != u_flat.size(0):
+        raise RuntimeError(f"{fn}: dout_flat must match u_flat shape")
     dim, dstate, mode = _common_checks(fn, u_flat, k_flat, cu_seqlens, max_seqlen, dt_idle, dt_active, A, B, C, D,
                                        tile_offsets, is_depthwise_bc, pw_B, pw_C, extra_cuda=(dout_flat, x),
                                        bwd=True, tile_chunk_size=tile_chunk_size)
     n_ch = int(cu_seqlens.size(0)) - 1
-    _check(x.dtype == torch.float32, f"{fn}: x must be float32")
-    _check(x.is_contiguous(), f"{fn}: x must be contiguous")
-    _check(x.dim() == 3 and x.size(0) == n_ch and x.size(2) == dstate * 2,
-           f"{fn}: x must have shape (n_channels, n_chunks, dstate*2)")
-    _check(x.size(1) == n_chunks_for(max_seqlen),
-           f"{fn}: x.size(1) must equal n_chunks = (max_seqlen + 2047) / 2048")
+    if x.dtype != torch.float32:
+        raise RuntimeError(f"{fn}: x must be float32")
+    if not (x.is_contiguous()):
+        raise RuntimeError(f"{fn}: x must be contiguous")
+    if not (x.dim() == 3 and x.size(0) == n_ch and x.size(2) == dstate * 2):
+        raise RuntimeError(f"{fn}: x must have shape (n_channels, n_chunks, dstate*2)")
+    if x.size(1) != n_chunks_for(max_seqlen):
+        raise RuntimeError(f"{fn}: x.size(1) must equal n_chunks = (max_seqlen + 2047) / 2048")
     has_z = z is not None
     if has_z:
-        _check(out is not None, f"{fn}: out (forward ungated output) must be provided when z is provided")
-        _check(z.dtype == u_flat.dtype and out.dtype == u_flat.dtype, f"{fn}: z/out must match u_flat dtype")
-        _check(z.is_cuda and out.is_cuda and z.is_contiguous() and out.is_contiguous(),
-               f"{fn}: z/out must be contiguous CUDA tensors")
-        _check(z.size(0) == u_flat.size(0) and out.size(0) == u_flat.size(0), f"{fn}: z/out must have shape (E,)")
+        if out is None:
+            raise RuntimeError(f"{fn}: out (forward ungated output) must be provided when z is provided")
+        if not (z.dtype == u_flat.dtype and out.dtype == u_flat.dtype):
+            raise RuntimeError(f"{fn}: z/out must match u_flat dtype")
+        if not (z.is_cuda and out.is_cuda and z.is_contiguous() and out.is_contiguous()):
+            raise RuntimeError(f"{fn}: z/out must be contiguous CUDA tensors")
+        if not (z.size(0) == u_flat.size(0) and out.size(0) == u_flat.size(0)):
+            raise RuntimeError(f"{fn}: z/out must have shape (E,)")
     dev = u_flat.device
     E = int(u_flat.size(0))
     f32 = dict(dtype=torch.float32, device=dev)
@@ -318,7 +364,7 @@ def bwd_flat_ch(u_flat, k_flat, cu_seqlens, max_seqlen, dt_idle, dt_active, A, B
     dD = torch.empty(dim, **f32) if D is not None else None
     dz = torch.empty_like(u_flat) if has_z else None
     dpw_B = dpw_C = None
-    with torch.cuda.device(dev):
+    with _nat.on_device(dev):
         s = _nat.stream_of(u_flat)
         if mode == "depthwise":
             W_B, W_C = (pw_B @ B, pw_C @ C) if pw_B is not None else (B, C)
@@ -364,9 +410,10 @@ def bwd_flat_ch(u_flat, k_flat, cu_seqlens, max_seqlen, dt_idle, dt_active, A, B
                 _nat.call("bcm_scan_bwd", a, s)
             else:
                 bitmask, mrd, tile_start, dx = _rows
-                _check(pw_B is None, f"{fn}: dense rows need W_B / W_C without pw_B / pw_C")
-                _check(dx.is_contiguous() and dx.dtype == u_flat.dtype and dx.dim() == 2
-                       and dx.size(0) == n_ch, f"{fn}: dx must be a contiguous (n_channels, L) tensor of u's dtype")
+                if not (pw_B is None):
+                    raise RuntimeError(f"{fn}: dense rows need W_B / W_C without pw_B / pw_C")
+                if not (dx.is_contiguous() and dx.dtype == u_flat.dtype and dx.dim() == 2 and dx.size(0) == n_ch):
+                    raise RuntimeError(f"{fn}: dx must be a contiguous (n_channels, L) tensor of u's dtype")
                 r = _nat.ScanRows()
                 r.bitmask, r.mask_row_div, r.tile_start = bitmask.data_ptr(), int(mrd), tile_start.data_ptr()
                 r.seqlen, r.dx = int(dx.size(1)), dx.data_ptr()

@@ -129,19 +129,6 @@ def selective_scan_flat_ch_fn(u_flat, k_flat, cu_seqlens, max_seqlen, dt_idle, d
     (selective_scan_interface.py:1182-1237). In depthwise mode B and C are
     the [dim, dstate] weights W_B / W_C; B[i,s] = u[i]*W_B[d,s] and
     C[i,s] = u[i]*W_C[d,s] are formed in the kernel. Returns (out, x)."""
-    u_flat, k_flat, cu_seqlens = u_flat.contiguous(), k_flat.contiguous(), cu_seqlens.contiguous()
-    dt_idle, dt_active = dt_idle.contiguous(), dt_active.contiguous()
-    A, B, C = A.contiguous(), B.contiguous(), C.contiguous()
-    if D is not None:
-        D = D.contiguous()
-    if z is not None:
-        z = z.contiguous()
-    if tile_offsets is not None:
-        tile_offsets = tile_offsets.contiguous()
-    if pw_B is not None:
-        pw_B = pw_B.contiguous()
-    if pw_C is not None:
-        pw_C = pw_C.contiguous()
     return SelectiveScanFlatChFn.apply(u_flat, k_flat, cu_seqlens, dt_idle, dt_active, A, B, C, D, z, max_seqlen,
                                        tile_offsets, tile_chunk_size, is_depthwise_bc, pw_B, pw_C)
 
