@@ -119,6 +119,9 @@ SIGNATURES = {
                              c_p]),
     "bcm_block_params_fwd": (c_i32, [c_p, c_p, c_p, c_p, c_i64, c_i64, c_f32, c_p, c_p, c_p, c_p, c_p, c_p]),
     "bcm_block_params_bwd": (c_i32, [c_p, c_p, c_p, c_i64, c_i64] + [c_p] * 10),
+    "bcm_residual_norm_fwd": (c_i32, [c_p, c_p, c_f32, c_p, c_p, c_i64, c_i64, c_f32] + [c_p] * 5),
+    "bcm_residual_norm_workspace_bytes": (c_i64, [c_i64, c_i64]),
+    "bcm_residual_norm_bwd": (c_i32, [c_p, c_p, c_p, c_f32, c_p, c_p, c_p, c_i64, c_i64] + [c_p] * 5 + [c_i64, c_p]),
 }
 
 RESTORE_BWD_NOALLOC_MAX_TILES = 699040  # BCM_RESTORE_BWD_NOALLOC_MAX_TILES of the header

@@ -23,7 +23,7 @@ LIBNAME = "libbcm_event_scan.so"
 ARCH = os.environ.get("BCM_OFFLOAD_ARCH", "gfx950")
 
 SOURCES = ["abi.hip", "extract.hip", "scan.hip", "scan_sl.hip", "scan_var.hip", "restore.hip", "restore_proj.hip", "conv.hip",
-           "gemm.hip", "params.hip"]
+           "gemm.hip", "params.hip", "rows.hip"]
 
 # Packed FP32 (v_pk_*_f32) generation is switched off for all device code.
 HIPCC_FLAGS = [

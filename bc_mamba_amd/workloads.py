@@ -117,8 +117,9 @@ class _ResidualPreNorm(torch.nn.Module):
         self.leak_alpha = leak_alpha
 
     def forward(self, s_in, v_in):
-        v_out = self.leak_alpha * v_in + self.core(s_in)
-        return self.core.to_spike(self.norm(v_out)), v_out
+        from .residual_norm import residual_norm
+        h, v_out = residual_norm(self.norm, v_in, self.core(s_in), self.leak_alpha)
+        return self.core.to_spike(h), v_out
 
 
 class SpikeMambaNet(torch.nn.Module):
@@ -151,11 +152,12 @@ class SpikeMambaNet(torch.nn.Module):
 
     def forward(self, tokens):
         from . import projections
+        from .residual_norm import layer_norm
         v = self.inp(tokens.long())
         s = self.in_spike(torch.sigmoid(projections.linear(v, self.in_prob.weight, self.in_prob.bias)))
         for blk in self.blocks:
             s, v = blk(s, v)
-        return self.head(self.norm(s).mean(dim=1))
+        return self.head(layer_norm(self.norm, s).mean(dim=1))
 
 
 def make_model_workload(seed=0, B=50, L=1024, device="cpu", **kw):

@@ -567,6 +567,23 @@ int bcm_block_params_bwd(const float* a0, const float* a1, const float* A, int64
                          const float* gA, const float* gB, const float* gC, float* da0,
                          float* da1, float* da_log, float* dw_bc, bcm_stream_t stream);
 
+/* ---- (6) leaky residual with its layer norm ------------------------------ */
+/* v_out = alpha v + dv and h = layer norm of v_out over its rows of D values
+ * (lra_impl.py:1381-1427), with the rows' mean and rstd for the backward; v
+ * NULL: h is the norm of dv, v_out is not written. The backward takes the gradients of
+ * h and of v_out (gv, NULL: zero): d_core is dv's, d_v v's (NULL: not written).
+ * All fp32, [rows, D] contiguous and 16-byte aligned, D a multiple of 4 up
+ * to 1024. */
+int bcm_residual_norm_fwd(const float* v, const float* dv, float alpha, const float* gamma,
+                          const float* beta, int64_t rows, int64_t D, float eps, float* v_out,
+                          float* h, float* mean, float* rstd, bcm_stream_t stream);
+int64_t bcm_residual_norm_workspace_bytes(int64_t rows, int64_t D);
+int bcm_residual_norm_bwd(const float* gh, const float* gv, const float* v_out, float alpha,
+                          const float* gamma, const float* mean, const float* rstd,
+                          int64_t rows, int64_t D, float* d_core, float* d_v, float* d_gamma,
+                          float* d_beta, void* workspace, int64_t workspace_bytes,
+                          bcm_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
