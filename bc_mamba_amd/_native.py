@@ -119,6 +119,10 @@ SIGNATURES = {
                              c_p]),
     "bcm_block_params_fwd": (c_i32, [c_p, c_p, c_p, c_p, c_i64, c_i64, c_f32, c_p, c_p, c_p, c_p, c_p, c_p]),
     "bcm_block_params_bwd": (c_i32, [c_p, c_p, c_p, c_i64, c_i64] + [c_p] * 10),
+    "bcm_spike_head_fwd": (c_i32, [c_p, c_i64, c_i64, c_i64, c_f32, c_p, c_p, c_p]),
+    "bcm_column_sums_workspace_bytes": (c_i64, [c_i64, c_i64]),
+    "bcm_column_sums": (c_i32, [c_p, c_i64, c_i64, c_p, c_p, c_i64, c_p]),
+    "bcm_spike_head_bwd": (c_i32, [c_p, c_p, c_i64, c_i64, c_p, c_p, c_p, c_i64, c_p]),
     "bcm_residual_norm_fwd": (c_i32, [c_p, c_p, c_f32, c_p, c_p, c_i64, c_i64, c_f32] + [c_p] * 5),
     "bcm_residual_norm_workspace_bytes": (c_i64, [c_i64, c_i64]),
     "bcm_residual_norm_bwd": (c_i32, [c_p, c_p, c_p, c_f32, c_p, c_p, c_p, c_i64, c_i64] + [c_p] * 5 + [c_i64, c_p]),

@@ -261,4 +261,7 @@ __device__ __forceinline__ float decay(float e) {
   return __builtin_amdgcn_exp2f(__builtin_amdgcn_fmed3f(e, -126.0f, 126.0f));
 }
 
+// torch's sigmoid of an fp32 value
+__device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
+
 }  // namespace bcm

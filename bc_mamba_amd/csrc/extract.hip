@@ -127,40 +127,48 @@ __global__ __launch_bounds__(256) void k_count(const T* __restrict__ x, int64_t 
 // e_model.py:233-254: s = (p >= thr) + p - p, evaluated left to right) on
 // p [B, L, Dm], writing the event bitmask of the rows (b, d) directly: no
 // transposed copy of s and no count pass over it. One wave per (b, 64
-// channels, 64-step tile): lane d reads p[b, l, d] for the tile's 64 steps
-// (each a coalesced 256-byte row of the wave), packs the 64 bits of its row
-// into one mask word pair and, when s is requested, writes s in p's layout.
-// Bits past L stay 0; the padding words of a row are not written.
-template <typename T>
+// channels, 32 steps): lane d reads p[b, l, d] for the 32 steps (each a
+// coalesced 256-byte row of the wave), packs the bits of its row into one mask
+// word and, when s is requested, writes s in p's layout. (With 64 steps a wave
+// 16000 x 128 values are 4 waves a CU: 11.0 us against 7.2; of logits, 51200 x
+// 256: 30.2 against 23.9. 16 steps: 8.3 and 25.1.)
+// Bits past L stay 0; the padding words of a row are not written. LOGITS: p
+// is given as its logits and taken through the sigmoid here, as torch
+// computes it: the probabilities are neither written nor read (16 + 21 -> 24 us
+// at 51200 x 256).
+constexpr int kSpikeT = 32;
+template <typename T, bool LOGITS>
 __global__ __launch_bounds__(256) void k_spike_bits(const T* __restrict__ p, int64_t B, int64_t L, int64_t Dm,
                                                     float thr, uint32_t* __restrict__ bitmask, int64_t W,
                                                     T* __restrict__ s_out) {
   const int lane = lane_id();
-  const int64_t nT = (L + kTile - 1) / kTile, nG = (Dm + kWave - 1) / kWave;
+  const int64_t nT = 2 * ((L + kTile - 1) / kTile), nG = (Dm + kWave - 1) / kWave;
   const int64_t gw = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
   if (gw >= B * nG * nT) return;
   const int64_t j = gw % nT, g = (gw / nT) % nG, b = gw / (nT * nG);
   const int64_t d = g * kWave + lane;
   if (d >= Dm) return;
-  const int64_t t0 = j * kTile;
-  const int n = (int)(L - t0 < kTile ? L - t0 : kTile);
+  const int64_t t0 = j * kSpikeT;
+  const int n = (int)(L - t0 < kSpikeT ? L - t0 : kSpikeT);  // below 1 in a last tile's second word
   const T* pr = p + (b * L + t0) * Dm + d;
   thr = to_f(from_f<T>(thr));  // torch compares in p's dtype
-  float v[kTile];
+  float v[kSpikeT];
 #pragma unroll
-  for (int l = 0; l < kTile; ++l) v[l] = l < n ? to_f(pr[(int64_t)l * Dm]) : 0.0f;  // all 64 loads in flight
-  uint32_t lo = 0, hi = 0;
+  for (int l = 0; l < kSpikeT; ++l) v[l] = l < n ? to_f(pr[(int64_t)l * Dm]) : 0.0f;  // all 32 loads in flight
+  if constexpr (LOGITS)
 #pragma unroll
-  for (int l = 0; l < kTile; ++l) {
+    for (int l = 0; l < kSpikeT; ++l) v[l] = sigmoid_f(v[l]);
+  uint32_t bits = 0;
+#pragma unroll
+  for (int l = 0; l < kSpikeT; ++l) {
     const bool hit = l < n && v[l] >= thr;
-    if (l < 32) lo |= (uint32_t)hit << l;
-    else hi |= (uint32_t)hit << (l - 32);
+    bits |= (uint32_t)hit << l;
   }
-  *reinterpret_cast<uint2*>(bitmask + (b * Dm + d) * W + 2 * j) = make_uint2(lo, hi);
+  bitmask[(b * Dm + d) * W + j] = bits;
   if (s_out) {
     T* sr = s_out + (b * L + t0) * Dm + d;
 #pragma unroll
-    for (int l = 0; l < kTile; ++l) {
+    for (int l = 0; l < kSpikeT; ++l) {
       if (l < n) {
         // the STE value rounded as torch rounds it: the hard spike in p's
         // dtype, plus p, minus p
@@ -835,23 +843,36 @@ int bcm_extract_fill_blocks_conv(const uint32_t* bitmask, const int32_t* counts,
   return check_launch(fn);
 }
 
-int bcm_spike_bits(const void* p, int dtype, int64_t B, int64_t L, int64_t Dm, float threshold, uint32_t* bitmask,
-                   void* s_out, bcm_stream_t stream) {
-  const char* fn = "bcm_spike_bits";
+static int spike_bits(const char* fn, bool logits, const void* p, int dtype, int64_t B, int64_t L, int64_t Dm,
+                      float threshold, uint32_t* bitmask, void* s_out, bcm_stream_t stream) {
   if (!dtype_ok(dtype)) return set_error(BCM_EINVAL, "%s: p must be fp32, fp16 or bf16", fn);
   if (B < 0 || L < 0 || Dm < 0) return set_error(BCM_EINVAL, "%s: negative size", fn);
   if (B == 0 || L == 0 || Dm == 0) return BCM_OK;
   if (!p || !bitmask) return set_error(BCM_EINVAL, "%s: null pointer", fn);
   if (!aligned(bitmask, 8)) return set_error(BCM_EINVAL, "%s: bitmask must be 8-byte aligned", fn);
   if (B * L * Dm > INT32_MAX) return set_error(BCM_EINVAL, "%s: B * L * Dm must fit in int32", fn);
-  const int64_t W = bitmask_words(L), nT = tile_count(L), nG = (Dm + kWave - 1) / kWave;
+  const int64_t W = bitmask_words(L), nT = 2 * tile_count(L), nG = (Dm + kWave - 1) / kWave;
   const dim3 grid(blocks_for(B * nG * nT, 4)), block(256);
-  dispatch_dtype(dtype, [&](auto tag) {
-    using T = decltype(tag);
-    hipLaunchKernelGGL((k_spike_bits<T>), grid, block, 0, hs(stream), static_cast<const T*>(p), B, L, Dm, threshold,
-                       bitmask, W, static_cast<T*>(s_out));
-  });
+  if (logits)
+    hipLaunchKernelGGL((k_spike_bits<float, true>), grid, block, 0, hs(stream), static_cast<const float*>(p), B, L, Dm,
+                       threshold, bitmask, W, static_cast<float*>(s_out));
+  else
+    dispatch_dtype(dtype, [&](auto tag) {
+      using T = decltype(tag);
+      hipLaunchKernelGGL((k_spike_bits<T, false>), grid, block, 0, hs(stream), static_cast<const T*>(p), B, L, Dm,
+                         threshold, bitmask, W, static_cast<T*>(s_out));
+    });
   return check_launch(fn);
+}
+
+int bcm_spike_bits(const void* p, int dtype, int64_t B, int64_t L, int64_t Dm, float threshold, uint32_t* bitmask,
+                   void* s_out, bcm_stream_t stream) {
+  return spike_bits("bcm_spike_bits", false, p, dtype, B, L, Dm, threshold, bitmask, s_out, stream);
+}
+
+int bcm_spike_head_fwd(const float* logits, int64_t B, int64_t L, int64_t Dm, float threshold, uint32_t* bitmask,
+                       float* s_out, bcm_stream_t stream) {
+  return spike_bits("bcm_spike_head_fwd", true, logits, BCM_F32, B, L, Dm, threshold, bitmask, s_out, stream);
 }
 
 int bcm_extract_count_bits(const uint32_t* bitmask, int64_t n_rows, int64_t L, int32_t* counts, int32_t* block_sums,

@@ -1,16 +1,18 @@
 // Row passes of the network around the blocks: the leaky residual with its
-// layer norm.
+// layer norm, and the gradient of a spike head's logits.
 //
 // Reference behaviour: lra_impl.py:1381-1427 (v' = alpha v + block(s),
-// h = norm(v')).
+// h = norm(v')), e_model.py:233-254 and :326-333 (p = sigmoid(logits), the
+// spikes pass p's gradient on).
 //
 // Bound by memory: what counts is how often a [tokens, D] array is read and
 // written. Torch runs the forward as three kernels over 7 arrays (17 + 24 + 54 us
 // at 51200 x 256) and the backward as six over 13 (50 + 50 + 5 us for the
 // norm, 24 + 17 us for the sum and the scaled gradient); here the forward is one
-// kernel over 4 arrays (35 us) and the backward one over 5 (43 us, with 7 for the
+// kernel over 4 arrays (33 us) and the backward one over 5 (40 us, and 5 for the
 // reduction of the workgroups' column sums): near 6 TB/s, part of it from the
-// last-level cache. D up to 1024, a row in the registers of at most one wave.
+// last-level cache. The head's gradient and its bias gradient take one kernel
+// and the reduction for torch's two (24 + 30 -> 26 + 5 us). D up to 1024, a row in the registers of at most one wave.
 #include "bcm_common.hpp"
 
 #include <algorithm>
@@ -91,8 +93,8 @@ __global__ __launch_bounds__(256) void k_residual_norm_fwd(const float* __restri
   if (at.lane == 0) mean[row] = mu, rstd[row] = rs;
 }
 
-// The workgroup's sums over its rows of acc (column sums, two of them: gamma's,
-// then beta's gradient) into part [2 D]; every thread comes here.
+// The workgroup's sums over its rows of acc (NA sets of column sums) into part
+// [NA D]; every thread comes here.
 template <int LP, int NV, int NA>
 __device__ __forceinline__ void column_sums(const RowAt<LP, NV>& at, const float4 (&acc)[NA][NV], float* part) {
   constexpr int G = 256 / LP, S = 4 * LP * NV;
@@ -160,6 +162,51 @@ __global__ __launch_bounds__(256) void k_residual_norm_bwd(const float* __restri
   column_sums<LP, NV, 2>(at, acc, part + (int64_t)blockIdx.x * 2 * D);
 }
 
+// d_logits = ds (1 - p) p with p = sigmoid(logits), rounded as torch rounds it;
+// part [workgroup][D]: the workgroup's share of the bias gradient.
+template <int LP, int NV>
+__global__ __launch_bounds__(256) void k_spike_head_bwd(const float* __restrict__ ds, const float* __restrict__ logits,
+                                                        int64_t rows, int D, float* __restrict__ d_logits,
+                                                        float* __restrict__ part) {
+  constexpr int G = 256 / LP;
+  const RowAt<LP, NV> at(D);
+  float4 acc[1][NV] = {};
+  auto grad = [](float g, float l) {
+    const float p = sigmoid_f(l);
+    return g * (1.0f - p) * p;
+  };
+  for (int64_t row = (int64_t)blockIdx.x * G + threadIdx.x / LP; row < rows; row += (int64_t)gridDim.x * G) {
+    float4 g[NV], l[NV];
+    at.load(g, ds + row * D);
+    at.load(l, logits + row * D);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      g[i] = make_float4(grad(g[i].x, l[i].x), grad(g[i].y, l[i].y), grad(g[i].z, l[i].z), grad(g[i].w, l[i].w));
+      acc[0][i].x += g[i].x, acc[0][i].y += g[i].y, acc[0][i].z += g[i].z, acc[0][i].w += g[i].w;
+    }
+    at.store(d_logits + row * D, g);
+  }
+  column_sums<LP, NV, 1>(at, acc, part + (int64_t)blockIdx.x * D);
+}
+
+// part [workgroup][D]: the workgroup's share of x's column sums, in k_spike_head_bwd's
+// order (the bias gradient is the same where torch computes the sigmoid's).
+template <int LP, int NV>
+__global__ __launch_bounds__(256) void k_column_sums(const float* __restrict__ x, int64_t rows, int D,
+                                                     float* __restrict__ part) {
+  constexpr int G = 256 / LP;
+  const RowAt<LP, NV> at(D);
+  float4 acc[1][NV] = {};
+  for (int64_t row = (int64_t)blockIdx.x * G + threadIdx.x / LP; row < rows; row += (int64_t)gridDim.x * G) {
+    float4 g[NV];
+    at.load(g, x + row * D);
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      acc[0][i].x += g[i].x, acc[0][i].y += g[i].y, acc[0][i].z += g[i].z, acc[0][i].w += g[i].w;
+  }
+  column_sums<LP, NV, 1>(at, acc, part + (int64_t)blockIdx.x * D);
+}
+
 // out0[c] (c < D), out1[c - D] = the sum over the workgroups' shares part [n][cols],
 // in a fixed order: 16 columns a workgroup, each summed by 64 threads.
 __global__ __launch_bounds__(1024) void k_column_reduce(const float* __restrict__ part, int n, int cols, int D,
@@ -168,6 +215,7 @@ __global__ __launch_bounds__(1024) void k_column_reduce(const float* __restrict_
   const int c = blockIdx.x * 16 + threadIdx.x % 16, r = threadIdx.x / 16;
   float v = 0.0f;
   if (c < cols)
+#pragma unroll 8
     for (int i = r; i < n; i += 64) v += part[(int64_t)i * cols + c];
   sm[r][threadIdx.x % 16] = v;
   __syncthreads();
@@ -256,6 +304,48 @@ int bcm_residual_norm_bwd(const float* gh, const float* gv, const float* v_out, 
   hipLaunchKernelGGL(k_column_reduce, dim3((unsigned)((2 * D + 15) / 16)), dim3(1024), 0, hs(stream), part, (int)wgs,
                      (int)(2 * D), (int)D, d_gamma, d_beta);
   return check_launch(fn);
+}
+
+int64_t bcm_column_sums_workspace_bytes(int64_t rows, int64_t D) {
+  return rows < 1 || D < 1 ? 0 : row_workgroups(rows, D) * D * (int64_t)sizeof(float);
+}
+
+// d_logits null: the column sums of x alone (logits null then)
+static int column_sums_of(const char* fn, const float* x, const float* logits, int64_t rows, int64_t D,
+                          float* d_logits, float* out, void* workspace, int64_t workspace_bytes,
+                          bcm_stream_t stream) {
+  if (int rc = row_check(fn, rows, D)) return rc;
+  const int64_t wgs = rows ? row_workgroups(rows, D) : 0;
+  if (!out || (rows && (!x || !workspace))) return set_error(BCM_EINVAL, "%s: null pointer", fn);
+  if (workspace_bytes < wgs * D * (int64_t)sizeof(float)) return set_error(BCM_EINVAL, "%s: workspace too small", fn);
+  for (const void* p : {(const void*)x, (const void*)logits, (const void*)d_logits})
+    if (!aligned16(p)) return set_error(BCM_EINVAL, "%s: arrays must be 16-byte aligned", fn);
+  float* part = static_cast<float*>(workspace);
+  if (rows)
+    row_form(D, [&](auto lp, auto nv) {
+      constexpr int LP = decltype(lp)::value, NV = decltype(nv)::value;
+      const dim3 grid((unsigned)wgs), block(256);
+      if (d_logits)
+        hipLaunchKernelGGL((k_spike_head_bwd<LP, NV>), grid, block, 0, hs(stream), x, logits, rows, (int)D, d_logits, part);
+      else hipLaunchKernelGGL((k_column_sums<LP, NV>), grid, block, 0, hs(stream), x, rows, (int)D, part);
+    });
+  int rc = check_launch(fn);
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_column_reduce, dim3((unsigned)((D + 15) / 16)), dim3(1024), 0, hs(stream), part, (int)wgs, (int)D,
+                     (int)D, out, out);
+  return check_launch(fn);
+}
+
+int bcm_column_sums(const float* x, int64_t rows, int64_t D, float* out, void* workspace, int64_t workspace_bytes,
+                    bcm_stream_t stream) {
+  return column_sums_of("bcm_column_sums", x, nullptr, rows, D, nullptr, out, workspace, workspace_bytes, stream);
+}
+
+int bcm_spike_head_bwd(const float* ds, const float* logits, int64_t rows, int64_t D, float* d_logits, float* d_bias,
+                       void* workspace, int64_t workspace_bytes, bcm_stream_t stream) {
+  const char* fn = "bcm_spike_head_bwd";
+  if (rows > 0 && (!logits || !d_logits)) return set_error(BCM_EINVAL, "%s: null pointer", fn);
+  return column_sums_of(fn, ds, logits, rows, D, d_logits, d_bias, workspace, workspace_bytes, stream);
 }
 
 }  // extern "C"

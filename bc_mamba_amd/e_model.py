@@ -43,6 +43,7 @@ try:
     from . import projections
     from . import selective_scan_cuda
     from .causal_conv1d import causal_conv1d_fn, conv1d_bwd_events
+    from .residual_norm import MAX_DIM, _dense, _plain_mode, _plain_module
     from .runtime_breakdown import cuda_stage
     from .selective_scan_interface import selective_scan_flat_ch_fn
 except ImportError:  # imported with this directory on sys.path
@@ -52,6 +53,7 @@ except ImportError:  # imported with this directory on sys.path
     import projections
     import selective_scan_cuda
     from causal_conv1d import causal_conv1d_fn, conv1d_bwd_events
+    from residual_norm import MAX_DIM, _dense, _plain_mode, _plain_module
     from runtime_breakdown import cuda_stage
     from selective_scan_interface import selective_scan_flat_ch_fn
 
@@ -365,6 +367,66 @@ class _SpikeBitsFn(torch.autograd.Function):
         return grad_s, None
 
 
+class _SpikeHeadFn(torch.autograd.Function):
+    """A spike head on x [B, L, K]: the logits' product, then the sigmoid and
+    the "ste" spikes with their event bitmask as one kernel
+    (bcm_spike_head_fwd); the probabilities are recomputed from the saved
+    logits in the backward, whose bias gradient rides along
+    (bcm_spike_head_bwd). Values and gradients are those of projections.linear,
+    torch.sigmoid and _SpikeBitsFn."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, threshold: float):
+        logits = projections.linear(x, weight, bias)
+        B, L, Dm = logits.shape
+        s = torch.empty_like(logits)
+        bitmask = torch.empty((B * Dm, _nat.bitmask_words(L)), dtype=torch.int32, device=x.device)
+        with _nat.on_device(x.device):
+            _nat.call("bcm_spike_head_fwd", logits.data_ptr(), B, L, Dm, threshold, bitmask.data_ptr(), s.data_ptr(),
+                      _nat.stream_of(x))
+        s._bcm_event_bits = (bitmask, threshold, s._version)
+        ctx.save_for_backward(x, weight, bias, logits)
+        return s
+
+    @staticmethod
+    def backward(ctx, grad_s):
+        x, weight, bias, logits = ctx.saved_tensors
+        x2 = x.reshape(-1, x.size(-1))
+        if torch.is_grad_enabled():  # a graph of the gradients is asked for: torch's operations
+            p = torch.sigmoid(F.linear(x2, weight, bias))
+            g = grad_s.reshape(p.shape) * (1.0 - p) * p
+            return (g @ weight).view(x.shape), g.t() @ x2, g.sum(0) if bias is not None else None, None
+        grad_s = _dense(grad_s)
+        rows, Dm = x2.size(0), logits.size(-1)
+        g = torch.empty((rows, Dm), dtype=logits.dtype, device=x.device)
+        db = torch.empty(Dm, dtype=logits.dtype, device=x.device)
+        with _nat.on_device(x.device):
+            nbytes = int(_nat.lib().bcm_column_sums_workspace_bytes(rows, Dm))
+            ws = torch.empty(nbytes // 4, dtype=torch.float32, device=x.device)
+            _nat.call("bcm_spike_head_bwd", grad_s.data_ptr(), logits.data_ptr(), rows, Dm, g.data_ptr(),
+                      db.data_ptr(), ws.data_ptr(), nbytes, _nat.stream_of(x))
+        dx = projections.mm(g, weight).view(x.shape) if ctx.needs_input_grad[0] else None
+        dw = projections.weight_grad(g, x2) if ctx.needs_input_grad[1] else None
+        return dx, dw, db if bias is not None else None, None
+
+
+def spike_head(x, weight, bias, sampler):
+    """sampler(sigmoid(x @ weight.T + bias)): one fused function
+    (_SpikeHeadFn) where sampler is a SpikeSamplerSurrogate that takes the
+    fused "ste" kernel, without hooks, and x [B, L, K] and the parameters are
+    contiguous fp32 on the GPU (the backward's kernel: outputs a multiple of 4
+    up to 1024)."""
+    if (_plain_module(sampler, SpikeSamplerSurrogate) and sampler.mode == "ste" and sampler.fused_bits
+            and x.dim() == 3 and x.is_cuda and 0 < x.numel() < 2 ** 31 and weight.dim() == 2
+            and weight.size(1) == x.size(2) and 4 <= weight.size(0) <= MAX_DIM and weight.size(0) % 4 == 0
+            and x.size(0) * x.size(1) * weight.size(0) < 2 ** 31 and (bias is None or bias.shape == weight.shape[:1])
+            and all(t is None or (type(t) in (torch.Tensor, nn.Parameter) and t.dtype == torch.float32
+                                  and t.device == x.device and t.is_contiguous()) for t in (x, weight, bias))
+            and _plain_mode()):
+        return _SpikeHeadFn.apply(x, weight, bias, float(sampler.threshold))
+    return sampler(torch.sigmoid(projections.linear(x, weight, bias)))
+
+
 def _event_bits_of(s, extract_threshold):
     """The bitmask a spike tensor carries, if it still describes s and the
     extraction's strict s > extract_threshold selects exactly the spikes:
@@ -453,6 +515,8 @@ class Mamba(nn.Module):
                                        device=device)
 
     def to_spike(self, out):
+        if self.fused_event_path and self.prob_activation == "sigmoid":
+            return spike_head(out, self.prob_head.weight, self.prob_head.bias, self.spike_sampler)
         logits = projections.linear(out, self.prob_head.weight, self.prob_head.bias) if self.fused_event_path \
             else self.prob_head(out)
         p = torch.sigmoid(logits) if self.prob_activation == "sigmoid" else torch.clamp(logits, 0.0, 1.0)

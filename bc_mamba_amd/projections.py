@@ -118,6 +118,22 @@ def weight_grad(g, x, tokens_first=True):
     return torch.bmm(gs, x.reshape(SPLIT, c, x.size(1))).sum(0)
 
 
+def column_sum(g):
+    """g.sum(0) of a 2-D g: the bias gradient of a projection."""
+    if (type(g) in _PLAIN and g.dtype == torch.float32 and g.is_cuda and 0 < g.numel() < _LIMIT
+            and 4 <= g.size(1) <= 1024 and g.size(1) % 4 == 0 and g.is_contiguous() and g.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled() and g.requires_grad) and not torch.compiler.is_compiling()):
+        rows, D = g.shape
+        out = torch.empty(D, dtype=g.dtype, device=g.device)
+        with _nat.on_device(g.device):
+            nbytes = int(_nat.lib().bcm_column_sums_workspace_bytes(rows, D))
+            ws = torch.empty(nbytes // 4, dtype=torch.float32, device=g.device)
+            _nat.call("bcm_column_sums", g.data_ptr(), rows, D, out.data_ptr(), ws.data_ptr(), nbytes,
+                      _nat.stream_of(g))
+        return out
+    return g.sum(0)
+
+
 class _LinearFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias):
@@ -136,7 +152,7 @@ class _LinearFn(torch.autograd.Function):
         g2 = gy.reshape(-1, gy.size(-1))
         dx = mm(g2, weight).view(x.shape) if ctx.needs_input_grad[0] else None
         dw = weight_grad(g2, x.reshape(-1, x.size(-1))) if ctx.needs_input_grad[1] else None
-        db = g2.sum(0) if ctx.has_bias and ctx.needs_input_grad[2] else None
+        db = column_sum(g2) if ctx.has_bias and ctx.needs_input_grad[2] else None
         return dx, dw, db
 
 

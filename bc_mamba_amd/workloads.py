@@ -151,10 +151,10 @@ class SpikeMambaNet(torch.nn.Module):
         self.head = torch.nn.Linear(d_model, num_classes)
 
     def forward(self, tokens):
-        from . import projections
+        from .e_model import spike_head
         from .residual_norm import layer_norm
         v = self.inp(tokens.long())
-        s = self.in_spike(torch.sigmoid(projections.linear(v, self.in_prob.weight, self.in_prob.bias)))
+        s = spike_head(v, self.in_prob.weight, self.in_prob.bias, self.in_spike)
         for blk in self.blocks:
             s, v = blk(s, v)
         return self.head(layer_norm(self.norm, s).mean(dim=1))

@@ -137,6 +137,15 @@ int bcm_extract_fill_blocks(const uint32_t* bitmask, const int32_t* counts,
  * of each bitmask row are not written. */
 int bcm_spike_bits(const void* p, int dtype, int64_t B, int64_t L, int64_t Dm, float threshold,
                    uint32_t* bitmask, void* s_out, bcm_stream_t stream);
+/* bcm_spike_bits on the fp32 logits of p, p = 1 / (1 + exp(-logits)), and its
+ * backward: d_logits = ds (1 - p) p over [rows, D] (rows = B * L, D = Dm; 16-byte
+ * aligned, D a multiple of 4 up to 1024) and its column sums d_bias [D] in
+ * bcm_column_sums' workspace and order. */
+int bcm_spike_head_fwd(const float* logits, int64_t B, int64_t L, int64_t Dm, float threshold,
+                       uint32_t* bitmask, float* s_out, bcm_stream_t stream);
+int bcm_spike_head_bwd(const float* ds, const float* logits, int64_t rows, int64_t D,
+                       float* d_logits, float* d_bias, void* workspace,
+                       int64_t workspace_bytes, bcm_stream_t stream);
 /* counts and block_sums of bcm_extract_count_blocks from a finished bitmask
  * (bcm_spike_bits), for bcm_extract_fill_blocks(_conv). */
 int bcm_extract_count_bits(const uint32_t* bitmask, int64_t n_rows, int64_t L, int32_t* counts,
@@ -567,7 +576,7 @@ int bcm_block_params_bwd(const float* a0, const float* a1, const float* A, int64
                          const float* gA, const float* gB, const float* gC, float* da0,
                          float* da1, float* da_log, float* dw_bc, bcm_stream_t stream);
 
-/* ---- (6) leaky residual with its layer norm ------------------------------ */
+/* ---- (6) leaky residual with its layer norm, column sums ----------------- */
 /* v_out = alpha v + dv and h = layer norm of v_out over its rows of D values
  * (lra_impl.py:1381-1427), with the rows' mean and rstd for the backward; v
  * NULL: h is the norm of dv, v_out is not written. The backward takes the gradients of
@@ -583,6 +592,12 @@ int bcm_residual_norm_bwd(const float* gh, const float* gv, const float* v_out, 
                           int64_t rows, int64_t D, float* d_core, float* d_v, float* d_gamma,
                           float* d_beta, void* workspace, int64_t workspace_bytes,
                           bcm_stream_t stream);
+
+/* out [D] = the column sums of x [rows, D] (fp32, 16-byte aligned, D a
+ * multiple of 4 up to 1024): a projection's bias gradient. */
+int64_t bcm_column_sums_workspace_bytes(int64_t rows, int64_t D);
+int bcm_column_sums(const float* x, int64_t rows, int64_t D, float* out, void* workspace,
+                    int64_t workspace_bytes, bcm_stream_t stream);
 
 #ifdef __cplusplus
 }
