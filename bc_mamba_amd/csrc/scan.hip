@@ -372,6 +372,179 @@ __global__ __launch_bounds__((kScanThreadsG<G, false>)) void k_scan_fwd(const bc
   }
 }
 
+// ---------------------------------------------------- forward, few channels
+// With fewer channels than the chip has lane groups k_scan_fwd leaves it idle
+// (512 channels of 1229 events: 512 waves, each a quarter full, five passes of 16
+// states in a row). Here a channel takes a whole workgroup: its 64-lane pass covers
+// up to 64 R events, and the states are split over the NS waves, which share
+// the staged items; each wave leaves its states' part of every item's sum in
+// LDS, where the waves add them up row by row for the output. What bounds
+// it is the chain load -> states -> sum of one or two passes. 512 channels of
+// 1229 events, 16 states, bf16: 67 -> 17 us; 128 of 315: 23 -> 7. 8 waves against 4
+// and 2 there at 64 states: 25, 29, 48 us.
+template <int R, int NS, typename T, bool HAS_Z>
+__global__ __launch_bounds__(NS* kWave) void k_scan_fwd_few(const bcm_scan_args a) {
+  constexpr int G = kWave, C = G * R, HR = R / 2, TS = G * (R + 1);
+  constexpr uint32_t SZ = sizeof(T);
+  const int N = a.dstate, tabk = tab_gaps(N);
+  const int ch = blockIdx.x, d = ch % a.dim;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), j = lane_id();
+  const int e0 = a.cu_seqlens[ch], n = a.cu_seqlens[ch + 1] - e0;
+
+  __shared__ float sT[kTabElems];
+  __shared__ float sAl[kTabMaxN], sWB[kTabMaxN], sWBC[kTabMaxN], carry[2 * kTabMaxN];
+  __shared__ float tile[TS];     // the items' u, transposed (tile_pos)
+  __shared__ float red[NS][TS];  // the waves' sums; red[0] holds the items' gaps before
+  float* tilek = red[0];
+  const int64_t E = a.n_events;
+  const __amdgpu_buffer_rsrc_t ru = buf_rsrc(a.u, E * SZ), rk = buf_rsrc(a.k, E * 4), ro = buf_rsrc(a.out, E * SZ);
+  const __amdgpu_buffer_rsrc_t rz = buf_rsrc(a.z, HAS_Z ? E * SZ : 0), roz = buf_rsrc(a.out_z, HAS_Z ? E * SZ : 0);
+  const __amdgpu_buffer_rsrc_t racc = buf_rsrc(a.acc, a.acc ? E * 4 : 0);
+  const int nck = a.n_chunks;
+  report_seqlen(a, n);
+
+  // A pass's items, row by row (item q G + j in row q), rows dealt to the waves.
+  // Items past the channel's events are padding: Δ = 0 below.
+  constexpr int QW = (R + NS - 1) / NS;  // rows of a wave
+  float rawu[QW];
+  int rawk[QW];
+  auto issue = [&](int c) {
+    const uint32_t eb = (uint32_t)(e0 + c * C) + (uint32_t)j;
+#pragma unroll
+    for (int i = 0; i < QW; ++i) {
+      const uint32_t e = eb + (uint32_t)((i * NS + wave) * G);
+      rawu[i] = buf_load<T>(ru, e * SZ);
+      rawk[i] = buf_load_i32(rk, e * 4u);
+    }
+  };
+  auto to_tiles = [&]() {
+#pragma unroll
+    for (int i = 0; i < QW; ++i) {
+      const int q = i * NS + wave;
+      if (R % NS == 0 || q < R) {
+        const int at = tile_pos<R>(q * G + j);
+        tile[at] = rawu[i];
+        tilek[at] = __int_as_float(rawk[i]);
+      }
+    }
+  };
+  if (n > 0) issue(0);
+  const float dti = a.dt_idle[d], dta = a.dt_active[d];
+  const float Dv = a.D ? a.D[d] : 0.0f;
+  for (int s = threadIdx.x; s < N; s += NS * kWave) {
+    const float wb = a.W_B[(int64_t)d * N + s];
+    sAl[s] = a.A[(int64_t)d * N + s] * kLog2e;
+    sWB[s] = wb;
+    sWBC[s] = wb * a.W_C[(int64_t)d * N + s];
+  }
+  build_decay_table(sT, a, d, dti, dta, NS * kWave);
+  if (n > 0) to_tiles();
+  const bool exact_blk = exact_products(sAl, N, dti, dta);  // also the barrier after the LDS set-up
+
+  const int gp = max(a.chunk_g_pass, R), g_rows = (a.max_seqlen + gp - 1) / gp;
+  const int s_lo = wave * N / NS, s_hi = (wave + 1) * N / NS;
+  const int nch = n > 0 ? (n + C - 1) / C : 0;
+  for (int c = 0; c < nch; ++c) {
+    const int cnt = min(n - c * C, C);
+    const int nv = cnt - j * R;
+    const uint32_t eb = (uint32_t)(e0 + c * C);
+    const int cend = min(n, (c + 1) * C), xc = (cend - 1) / kXChunk;
+    const bool xsave = (cend % kXChunk == 0 || cend == n) && xc < nck;
+    if (c > 0) {
+      to_tiles();
+      __syncthreads();
+    }
+    if (c + 1 < nch) issue(c + 1);
+    const float* mine = tile + j * (R + 1);
+    const float* minek = tilek + j * (R + 1);
+    float dl[R], du2[R], acc[R];
+    uint32_t tb[R];
+    int big = 0;
+    float Sa = 0.0f, Sb = 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const bool valid = r < nv;
+      const int km1 = valid ? __float_as_int(minek[r]) - 1 : -1;
+      dl[r] = valid ? fmaf(dti, (float)km1, dta) : 0.0f;
+      const float uv = mine[r];
+      du2[r] = dl[r] * uv * uv;
+      tb[r] = (uint32_t)(km1 + 1) * 4u;
+      big |= km1 >= tabk ? 1 : 0;
+      if (r < HR) Sa += dl[r];
+      else Sb += dl[r];
+      acc[r] = 0.0f;
+    }
+    // the state before the backward's passes (gp events, a multiple of R)
+    const int gi = c * C + j * R;
+    const bool gsave = a.chunk_g && gi > 0 && gi < n && gi % gp == 0 && gi / gp < g_rows;
+    const int64_t grow = (int64_t)ch * g_rows + gi / gp;
+    auto states = [&](auto exact_tag) {
+      constexpr bool EXACT = decltype(exact_tag)::value;
+#pragma unroll 1
+      for (int s = s_lo; s < s_hi; ++s) {
+        const float Al = sAl[s], wbc = sWBC[s];
+        const uint32_t row = (uint32_t)(s * (tabk + 1) * 4);
+        float av[R], Pa = 1.0f, Ha = 0.0f, Pb = 1.0f, Hb = 0.0f;
+#pragma unroll
+        for (int r = 0; r < R; ++r) av[r] = EXACT ? decay(dl[r] * Al) : tab(sT, row, tb[r]);
+#pragma unroll
+        for (int i = 0; i < HR; ++i) {
+          Ha = fmaf(av[i], Ha, du2[i]);
+          Hb = fmaf(av[i + HR], Hb, du2[i + HR]);
+          if (EXACT) Pa *= av[i], Pb *= av[i + HR];
+        }
+        if (!EXACT) Pa = decay(Sa * Al), Pb = decay(Sb * Al);
+        float P = Pa * Pb, H = fmaf(Pb, Ha, Hb);
+        Wave64::scan_up(P, H);
+        const float g0 = c > 0 ? carry[N + s] : 0.0f, P0 = c > 0 ? carry[s] : 1.0f;
+        const float gend = fmaf(P, g0, H);
+        float ga = Wave64::prev(gend, g0), gb = fmaf(Pa, ga, Ha);
+        if (gsave) a.chunk_g[grow * N + s] = ga * sWB[s];
+#pragma unroll
+        for (int i = 0; i < HR; ++i) {
+          ga = fmaf(av[i], ga, du2[i]);
+          gb = fmaf(av[i + HR], gb, du2[i + HR]);
+          acc[i] = fmaf(ga, wbc, acc[i]);
+          acc[i + HR] = fmaf(gb, wbc, acc[i + HR]);
+        }
+        if (j == G - 1) {
+          const float Pn = P0 * P;
+          carry[s] = Pn;
+          carry[N + s] = gend;
+          if (xsave) reinterpret_cast<float2*>(a.x + ((int64_t)ch * nck + xc) * 2 * N)[s] = make_float2(Pn, gend * sWB[s]);
+        }
+      }
+    };
+    if (exact_blk || __any(big)) states(std::true_type{});
+    else states(std::false_type{});
+    __syncthreads();  // every wave has read the gaps
+#pragma unroll
+    for (int r = 0; r < R; ++r) red[wave][j * (R + 1) + r] = acc[r];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < QW; ++i) {
+      const int q = i * NS + wave;
+      if (R % NS != 0 && q >= R) break;
+      const int idx = q * G + j, at = tile_pos<R>(idx);
+      float sum = red[0][at];
+#pragma unroll
+      for (int w = 1; w < NS; ++w) sum += red[w][at];
+      const float uv = tile[at], yv = fmaf(Dv, uv, uv * sum);
+      const uint32_t off = idx < cnt ? (eb + idx) * SZ : kBufOOB;
+      buf_store<T>(ro, off, yv);
+      if (HAS_Z) {
+        const float zv = buf_load<T>(rz, off);
+        buf_store<T>(roz, off, yv * (zv / (1.0f + __expf(-zv))));
+      }
+      if (a.acc) buf_store_f32(racc, idx < cnt ? (eb + idx) * 4u : kBufOOB, sum);
+    }
+    __syncthreads();  // the tiles are written anew
+  }
+  // chunks past the channel's end keep the reference's zero state
+  for (int i = (max(n, 0) + kXChunk - 1) / kXChunk * 2 * N + threadIdx.x; i < nck * 2 * N; i += NS * kWave)
+    a.x[(int64_t)ch * nck * 2 * N + i] = 0.0f;
+}
+
 template <int G, int R, typename T, bool HAS_Z, bool TBL, bool DXR>
 __global__ __launch_bounds__((kScanThreadsG<G, true>)) void k_scan_bwd(const bcm_scan_args a, const ScanRows rw, int nw, int S) {
   using Ops = Grp<G>;
@@ -1095,6 +1268,34 @@ static bool rows_fusable(const bcm_scan_args& a, const bcm_scan_rows& r) {
   return r.seqlen % 4 == 0 && p % (4 * dtype_size(a.dtype)) == 0;
 }
 
+// Waves per channel of k_scan_fwd_few (0: k_scan_fwd): one for each state, up
+// to 8. Its work grows with channels x states from about 1024 channels on, while
+// k_scan_fwd then only fills its lanes: 2048 channels of 1230 events, four a
+// model channel, take 63 us there and 47 here at 16 states, 191 and 86 at 64, but
+// 38 and 38 at 8 and 26 and 32 at 4; 3000 channels 62 and 68 at 16. 1024 channels:
+// 57 and 26 at 16 states.
+static int few_waves(const bcm_scan_args& a) {
+  if (a.dstate > kTabMaxN || a.n_events == 0 || a.n_channels > (a.dstate >= 16 ? 2048 : 1024)) return 0;
+  if (a.chunk_g && a.chunk_g_pass % 16 != 0) return 0;
+  return a.dstate >= 8 ? 8 : a.dstate >= 4 ? 4 : a.dstate >= 2 ? 2 : 0;
+}
+
+template <typename T, bool Z> static int launch_few(const bcm_scan_args& a, int ns, hipStream_t s, const char* fn) {
+  auto go = [&](auto r, auto w) {
+    constexpr int R = decltype(r)::value, NS = decltype(w)::value;
+    hipLaunchKernelGGL((k_scan_fwd_few<R, NS, T, Z>), dim3((unsigned)a.n_channels), dim3(NS * kWave), 0, s, a);
+  };
+  auto waves = [&](auto r) {
+    if (ns == 8) go(r, std::integral_constant<int, 8>{});
+    else if (ns == 4) go(r, std::integral_constant<int, 4>{});
+    else go(r, std::integral_constant<int, 2>{});
+  };
+  if (a.max_seqlen <= 256) waves(std::integral_constant<int, 4>{});
+  else if (a.max_seqlen <= 512) waves(std::integral_constant<int, 8>{});
+  else waves(std::integral_constant<int, 16>{});
+  return check_launch(fn);
+}
+
 template <bool BWD>
 static int scan_entry(const bcm_scan_args* ap, bcm_stream_t stream, const char* fn, const ScanRows* rw = nullptr) {
   if (!ap) return set_error(BCM_EINVAL, "%s: null args", fn);
@@ -1149,6 +1350,12 @@ static int scan_entry(const bcm_scan_args* ap, bcm_stream_t stream, const char* 
   int rc = BCM_OK;
   dispatch_dtype(a.dtype, [&](auto tag) {
     using T = decltype(tag);
+    if constexpr (!BWD) {
+      if (const int ns = few_waves(a)) {
+        rc = z ? launch_few<T, true>(a, ns, s, fn) : launch_few<T, false>(a, ns, s, fn);
+        return;
+      }
+    }
     rc = z ? dispatch_shape<T, true, BWD>(a, s, fn, nullptr, rw) : dispatch_shape<T, false, BWD>(a, s, fn, nullptr, rw);
   });
   return rc;

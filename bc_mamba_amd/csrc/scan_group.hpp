@@ -144,4 +144,18 @@ template <> struct Grp<32> {
   }
 };
 
+// The whole wave: the forward steps of Grp<32>, then rows 2 and 3 combine with
+// lane 31 (DPP row_bcast:31). Only what the forward needs; the backward's
+// 64-lane groups use the generic form.
+struct Wave64 {
+  static __device__ __forceinline__ void scan_up(float& P, float& H) {
+    Grp<32>::scan_up(P, H);
+    asm("s_nop 1\n\tv_fmac_f32_dpp %0, %0, %1 row_bcast:31 row_mask:0xc bank_mask:0xf" : "+v"(H) : "v"(P));
+    asm("s_nop 1\n\tv_mul_f32_dpp %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf" : "+v"(P));
+  }
+  static __device__ __forceinline__ float prev(float v, float first) {  // lane j-1; `first` in lane 0
+    return dpp_mov<0x138>(v, first);                                    // wave_shr:1
+  }
+};
+
 }  // namespace bcm
