@@ -12,8 +12,8 @@ events and builds the event index, the restore reads that index instead of
 rebuilding it, the scan backward writes the dense x_conv gradient rows from
 the same index (no separate gather backward), and the per-block host syncs
 drop from two to one. The fused path's token projections (in_proj, out_proj,
-prob_head) take their weight gradients as split-K products
-(`projections`). With `conv_at_events=True` (default) the depthwise
+prob_head) run on this package's fp32 product (`projections`), the spike head
+as one function (`spike_head`). With `conv_at_events=True` (default) the depthwise
 conv + SiLU is evaluated only at the events, by the extraction itself, and
 its backward goes from du straight to the conv input's gradient: no dense
 x_conv exists in either direction. With `fused_out_proj=True` (default; fp32)
@@ -253,8 +253,8 @@ class _IndexedRestoreProjFn(torch.autograd.Function):
     one kernel that computes dz tile by tile on the matrix cores and runs
     the restore backward's sweep on it (bcm_restore_proj_bwd).
 
-    mode "gemm": z is formed for the forward GEMM (and again for the weight
-    gradient's split-K GEMM) and freed, hipBLASLt runs the two products.
+    mode "gemm": z is formed for the forward product (and again for the weight
+    gradient's) and freed, projections.mm and weight_grad run the two.
     mode "mfma": the forward and the weight gradient also run as this
     package's kernels, with z generated from the event index inside them
     (bcm_restore_proj_fwd, bcm_restore_proj_bwd): no dense z at all.
