@@ -162,6 +162,18 @@ def call(name, *args):
         raise RuntimeError(lib().bcm_last_error().decode())
 
 
+_wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+_legacy_batched = torch._C._functorch.is_legacy_batchedtensor
+
+
+def no_memory(*tensors):
+    """One of the tensors (None among them is passed over) stands for several
+    and has no memory of its own: a batched gradient
+    (torch.autograd.grad(..., is_grads_batched=True), vmap over a backward).
+    Its type is torch.Tensor's all the same."""
+    return any(t is not None and (_wrapped(t) or _legacy_batched(t)) for t in tensors)
+
+
 def ptr(t):
     return None if t is None else t.data_ptr()
 

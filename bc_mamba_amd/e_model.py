@@ -334,7 +334,8 @@ class _BlockParamsFn(torch.autograd.Function):
     def backward(ctx, *grads):
         a0, a1, A = ctx.saved_tensors
         D, N = A.shape
-        if torch.is_grad_enabled():  # a graph of the gradients is asked for: torch's operations
+        if torch.is_grad_enabled() or _nat.no_memory(*grads):
+            # a graph of the gradients is asked for, or a batch of them at once: torch's operations
             gi, ga, gA, gB, gC = (A.new_zeros(s) if g is None else g
                                   for g, s in zip(grads, (D, D, (D, N), (D, N), (D, N))))
             # softplus' derivative, 1 past its threshold
@@ -392,7 +393,8 @@ class _SpikeHeadFn(torch.autograd.Function):
     def backward(ctx, grad_s):
         x, weight, bias, logits = ctx.saved_tensors
         x2 = x.reshape(-1, x.size(-1))
-        if torch.is_grad_enabled():  # a graph of the gradients is asked for: torch's operations
+        if torch.is_grad_enabled() or _nat.no_memory(grad_s):
+            # a graph of the gradients is asked for, or a batch of them at once: torch's operations
             p = torch.sigmoid(F.linear(x2, weight, bias))
             g = grad_s.reshape(p.shape) * (1.0 - p) * p
             return (g @ weight).view(x.shape), g.t() @ x2, g.sum(0) if bias is not None else None, None

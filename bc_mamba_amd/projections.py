@@ -47,12 +47,12 @@ def _major(t, rows, cols):
 def _kernel_form(x, y, bias=None):
     """The kernel's operand forms for x @ y (+ bias), or None where the
     product stays with torch: other types and devices, a product that
-    autograd must see (no custom backward around it), autocast, a traced or
-    wrapped tensor, strides without a contiguous dimension, an operand of 2 GiB."""
+    autograd must see (no custom backward around it), autocast, a traced,
+    wrapped or batched tensor, strides without a contiguous dimension, an operand of 2 GiB."""
     grad = torch.is_grad_enabled()
     for t in (x, y) if bias is None else (x, y, bias):
         if (type(t) not in _PLAIN or t.dtype != torch.float32 or not t.is_cuda or t.device != x.device
-                or (grad and t.requires_grad)):
+                or (grad and t.requires_grad) or _nat.no_memory(t)):
             return None
     if torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling():
         return None
@@ -121,7 +121,8 @@ def weight_grad(g, x, tokens_first=True):
 def column_sum(g):
     """g.sum(0) of a 2-D g: the bias gradient of a projection."""
     if (type(g) in _PLAIN and g.dtype == torch.float32 and g.is_cuda and 0 < g.numel() < _LIMIT
-            and 4 <= g.size(1) <= 1024 and g.size(1) % 4 == 0 and g.is_contiguous() and g.data_ptr() % 16 == 0
+            and 4 <= g.size(1) <= 1024 and g.size(1) % 4 == 0 and g.is_contiguous()
+            and not _nat.no_memory(g) and g.data_ptr() % 16 == 0
             and not (torch.is_grad_enabled() and g.requires_grad) and not torch.compiler.is_compiling()):
         rows, D = g.shape
         out = torch.empty(D, dtype=g.dtype, device=g.device)

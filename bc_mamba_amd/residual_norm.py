@@ -79,7 +79,8 @@ class _ResidualNormFn(torch.autograd.Function):
     def backward(ctx, gh, gv):
         x, weight, mean, rstd = ctx.saved_tensors
         alpha, residual = ctx.alpha, ctx.residual
-        if gh is None or torch.is_grad_enabled():  # the residual alone, or a graph of the gradients is asked for
+        # the residual alone, a graph of the gradients asked for, or a batch of gradients at once
+        if gh is None or torch.is_grad_enabled() or _nat.no_memory(gh, gv):
             d, dw, db = gv, None, None
             if gh is not None:
                 mu = x.mean(-1, keepdim=True)
