@@ -239,7 +239,7 @@ template <typename F> static bool row_form(int64_t D, F&& f) {
   return false;
 }
 
-// Workgroups of a backward pass: eight a CU at most.
+// Workgroups of a backward pass: four a CU at most.
 static int64_t row_workgroups(int64_t rows, int64_t D) {
   int64_t G = 1;
   row_form(D, [&](auto lp, auto) { G = 256 / decltype(lp)::value; });
